@@ -304,6 +304,8 @@ hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, 
         return path == IQ_PATH_AUTO && !isum ? launch_float_mm(v, x, w->cols, m, y, w->rows, s) : hipErrorNotSupported;
     if (path == IQ_PATH_AUTO) {
         if (!isum && dense_mfma_supported(v, m)) e = launch_dense_mfma(v, x, w->cols, m, y, w->rows, ws, s);
+        if (e == hipErrorNotSupported && !isum && q8_tile_supported(v, m))
+            e = launch_q8_tile(v, x, w->cols, m, y, w->rows, ws, s);
         if (e == hipErrorNotSupported && !isum && gemv_supported(v, m)) e = launch_gemv(v, x, w->cols, m, y, w->rows, s);
     } else if (path == IQ_PATH_GEMV) {
         e = launch_gemv(v, x, w->cols, m, y, w->rows, s);

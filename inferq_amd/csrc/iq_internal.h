@@ -84,6 +84,12 @@ hipError_t launch_dense_mfma(const WeightView& w, const float* x, int64_t ldx, i
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
                                  void* ws, hipStream_t s);
 
+// Q8_0 matrices at many input rows on f16 MFMA in the exact lane order
+// (iq_q8_tile.hip); quantises x itself into `ws` (at least act_bytes).
+bool q8_tile_supported(const WeightView& w, int64_t m);
+hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
+                          hipStream_t s);
+
 // y[m][ldy] = x . W^T for F32 and BF16 matrices (iq_dense_f32.hip), in the
 // MoE router's f32 order; hipErrorNotSupported for other dtypes.
 hipError_t launch_float_mm(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,

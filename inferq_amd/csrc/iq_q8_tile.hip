@@ -1,0 +1,274 @@
+// iq_q8_tile.hip -- y = x . W^T for Q8_0 matrices at many input rows (prefill
+// widths), in the reference's exact per-lane order (q80_tile,
+// src/qgemm.rs:369-397): every output is bitwise the one-row result.
+//
+// The reference's lane k owns bytes 4k..4k+3 of every 32-value block and
+// advances acc_k = fma(f16(dw) * f16(dx), dot4_k, acc_k) once per block; the
+// eight lanes meet in hsum_f32_8.  v_mfma_f32_16x16x4_4b_f16 multiplies four
+// independent 16 x 4 by 4 x 16 pairs, which is dot4_k of a 16 x 16 tile for
+// four lanes k at once: two of them per block give all eight.  The int8
+// values are exact in f16, a product is at most 2^14 and a dot at most 2^16,
+// so the f32 results are the exact integers, already converted.
+//
+// What bounds it: the chains.  Each output takes eight FMAs and one scale
+// product per 32 values, 9 VALU issues where a dot of 32 values is 1/16 of
+// an int8 MFMA; on [512 x 4096] -> 2048 that is 31 us of VALU issue at
+// 2.4 GHz, and the MFMAs another 15.
+#include "iq_internal.h"
+#include "iq_quant.h"
+
+namespace iq {
+
+namespace {
+
+typedef _Float16 v4h __attribute__((ext_vector_type(4)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+constexpr int kQtCols = 64;  // weight rows per workgroup (16 per wave)
+constexpr int kQtRows = 32;  // input rows per workgroup (16 per wave)
+constexpr int kQtCB = 4;     // 32-value blocks per LDS stage
+
+struct QtArgs {
+    const uint8_t* w;  // [n][row_bytes], 4-byte aligned rows
+    int64_t n, row_bytes;
+    int nb;            // 32-value blocks per row, a multiple of kQtCB
+    const int8_t* q;   // [m][nb * 32] quantised x, natural order
+    const float* d;    // [m][nb] block scales
+    int m;
+    float* y;  // [m][ldy]
+    int64_t ldy;
+};
+
+// One wave per (row, 256 values): Q8_0 (bit-exact from_float).  The bytes
+// are stored + 128, the form bytes_to_f16 takes.
+__global__ __launch_bounds__(256) void k_qt_quant(const float* __restrict__ x, int64_t ldx, int64_t m, int64_t k,
+                                                  int8_t* __restrict__ q, float* __restrict__ d) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int ng = (int)((k + 255) / 256);
+    if (wid >= m * ng) return;  // uniform per wave
+    const int64_t row = wid / ng;
+    const int g = (int)(wid - row * ng);
+    const Q80Lane r = quant_q80_core(q80_vals4_load(x + row * ldx, k, g));
+    const int64_t b = (int64_t)g * 8 + (lane >> 3);
+    if (b >= k / 32) return;
+    ((uint32_t*)(q + row * k + (int64_t)g * 256))[lane] = r.packed ^ 0x80808080u;
+    if ((lane & 7) == 0) d[row * (k / 32) + b] = f16_to_f32(r.dh);
+}
+
+// Four bytes u as f16 values u - 128: the bytes under the exponent of 1024, less 1152.
+__device__ __forceinline__ u32x2 bytes_to_f16(uint32_t u) {
+    const v2h off = {(_Float16)-1152.f, (_Float16)-1152.f};
+    const v2h lo = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) + off;
+    const v2h hi = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) + off;
+    return u32x2{__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi)};
+}
+
+// LDS stage of kQtCB blocks: A f16 [block][32 rows][64 bytes], B the same of
+// the 64 weight rows, D the rows' block scales, W the weight rows'.  The 16
+// bytes p of a row's 64 hold the dwords of reference lanes p and p + 4, what
+// lane group p of a fragment multiplies.  Block planes are padded so that the
+// four blocks one row's threads park go to different banks.
+struct QtStage {
+    static constexpr int AP = kQtRows * 64 + 16, BP = kQtCols * 64 + 16;
+    static constexpr int A = 0;
+    static constexpr int B = A + kQtCB * AP;
+    static constexpr int D = B + kQtCB * BP;
+    static constexpr int W = D + kQtCB * kQtRows * 4;
+    static constexpr int END = W + kQtCB * kQtCols * 4;
+};
+
+// Grid (n / 64, m / 32): wave w has weight rows 16 (w % 4) .. +15 and input
+// rows 16 (w / 4) .. +15.  One 16 x 16 tile per wave (32 chains) leaves four
+// waves per SIMD, which VALU issue needs: on this chip a wave alone issues an
+// f32 FMA every 5 cycles, two or four of them one every 2.7 together.  [512 x
+// 4096] -> 2048 / [200 x 4096] -> 2048 / [333 x 2048] -> 4096: 60 / 37 / 44 us
+// (the lane kernel: 243 / 124 / 148); 64 rows per workgroup 61 / 53 / 54; 16
+// rows 77 / 44 / 53; two tiles per wave with the MFMAs issued one step ahead,
+// two waves per SIMD, 61 / 54 / 56; a second stage of loads in flight the same;
+// every thread staging a quarter block (narrower loads, three times as many)
+// 68 / 45 / 52.
+__global__ __launch_bounds__(512, 4) void k_qt_mm(QtArgs a) {
+    constexpr int R = kQtRows, NT = 512;
+    using L = QtStage;
+    __shared__ __align__(16) uint8_t st[2][L::END];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, jj = lane & 15;
+    const int rbase = (wave >> 2) * 16, cbase = (wave & 3) * 16;
+    const int64_t n0 = (int64_t)blockIdx.x * kQtCols;
+    const int row0 = (int)blockIdx.y * R;
+    const int rows = min(R, a.m - row0);
+
+    // ---- staging, a block of a row per item: the first four waves take the
+    // weight rows, the last ones the input rows, in registers of their own
+    // (shared ones would make the waves wait for the loads where the
+    // branches join)
+    constexpr int kB = kQtCols * kQtCB, kA = R * kQtCB;
+    static_assert(kB == 256 && kA == 128, "items of whole waves");
+    const int tb = threadIdx.x, ta = NT - 1 - (int)threadIdx.x;
+    const bool hasb = tb < kB, hasa = ta < kA;
+    const int bc = tb & 3, ac = ta & 3, bcl = (tb >> 2) & (kQtCols - 1), arl = (ta >> 2) & (R - 1);
+    const uint8_t* bsrc = a.w + min(n0 + bcl, a.n - 1) * a.row_bytes + 34 * bc;
+    // quants from the aligned dword at or before them: an even block's start
+    // two bytes into it (the ninth dword's upper half is the next block's),
+    // an odd block's at it
+    const int bodd = bc & 1;
+    const int64_t arow = row0 + min(arl, rows - 1);
+    const int8_t* asrc = a.q + (arow * a.nb + ac) * 32;
+    const float* dsrc = a.d + arow * a.nb + ac;
+
+    u32x4 b0 = {}, b1 = {}, a0 = {}, a1 = {};
+    uint32_t b2 = 0, bw = 0;  // the ninth dword, the scale
+    float ad = 0.f;
+    auto issue = [&](int s) {
+        if (hasb) {
+            const uint8_t* p = bsrc + (int64_t)s * (34 * kQtCB);
+            const uint8_t* pq = p + 2 * bodd;
+            b0 = *(const u32x4*)pq;
+            b1 = *(const u32x4*)(pq + 16);
+            b2 = ld32(pq + (bodd ? 28 : 32));
+            bw = ld16(p);
+        }
+        if (hasa) {
+            const int8_t* p = asrc + (int64_t)s * (32 * kQtCB);
+            a0 = *(const u32x4*)p;
+            a1 = *(const u32x4*)(p + 16);
+            ad = dsrc[(int64_t)s * kQtCB];
+        }
+    };
+    // 16 bytes p of a row's 64: dwords p and p + 4 as f16
+    auto park_block = [&](uint8_t* dst, const uint32_t (&v)[8]) {
+#pragma unroll
+        for (int p = 0; p < 4; p++) {
+            const u32x2 lo = bytes_to_f16(v[p]), hi = bytes_to_f16(v[p + 4]);
+            *(u32x4a16*)(dst + 16 * p) = u32x4a16{lo.x, lo.y, hi.x, hi.y};
+        }
+    };
+    auto park = [&](int P) {
+        if (hasb) {
+            const uint32_t w[9] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w, b2};
+            const uint32_t sh = bodd ? 0u : 2u;
+            uint32_t v[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], sh) ^ 0x80808080u;
+            park_block(st[P] + L::B + bc * L::BP + bcl * 64, v);
+            *(float*)(st[P] + L::W + 4 * (bc * kQtCols + bcl)) = f16_to_f32(bw);
+        }
+        if (hasa) {
+            const uint32_t v[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+            park_block(st[P] + L::A + ac * L::AP + arl * 64, v);
+            *(float*)(st[P] + L::D + 4 * (ac * R + arl)) = ad;
+        }
+    };
+
+    // acc[k][r]: chain of reference lane k, output (row 4 q + r, column jj) of the wave's tile
+    float acc[8][4];
+#pragma unroll
+    for (int k = 0; k < 8; k++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) acc[k][r] = 0.f;
+
+    const int ns = a.nb / kQtCB;
+    issue(0);
+    park(0);
+    lds_barrier();
+    for (int s = 0; s < ns; s++) {
+        const uint8_t* S = st[s & 1];
+        if (s + 1 < ns) issue(s + 1);
+        // A (row jj) and B (column jj) of 16x16x4: lane group q holds the
+        // four values of its block q.  A block's operands are read while the
+        // one before it is multiplied.
+        struct Frag {
+            u32x4a16 a, b;
+            f32x4 yd;
+            float xd;
+        };
+        auto load = [&](int c) {
+            return Frag{*(const u32x4a16*)(S + L::A + c * L::AP + (rbase + jj) * 64 + 16 * q),
+                        *(const u32x4a16*)(S + L::B + c * L::BP + (cbase + jj) * 64 + 16 * q),
+                        *(const f32x4*)(S + L::D + 4 * (c * R + rbase + 4 * q)),
+                        *(const float*)(S + L::W + 4 * (c * kQtCols + cbase + jj))};
+        };
+        Frag f = load(0);
+        if (rbase < rows)  // uniform per wave
+#pragma unroll
+        for (int c = 0; c < kQtCB; c++) {
+            const v16f z = {};
+            const v16f d0 = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4h, u32x2{f.a.x, f.a.y}),
+                                                                 __builtin_bit_cast(v4h, u32x2{f.b.x, f.b.y}), z, 0, 0, 0);
+            const v16f d1 = __builtin_amdgcn_mfma_f32_16x16x4f16(__builtin_bit_cast(v4h, u32x2{f.a.z, f.a.w}),
+                                                                 __builtin_bit_cast(v4h, u32x2{f.b.z, f.b.w}), z, 0, 0, 0);
+            const float dd[4] = {f.xd * f.yd.x, f.xd * f.yd.y, f.xd * f.yd.z, f.xd * f.yd.w};
+            if (c + 1 < kQtCB) f = load(c + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[k][r] = __builtin_fmaf(dd[r], d0[4 * k + r], acc[k][r]);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[k + 4][r] = __builtin_fmaf(dd[r], d1[4 * k + r], acc[k + 4][r]);
+            // the chains are advanced here, not sunk, which bounds the live MFMA results
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) asm volatile("" : "+v"(acc[k][r]));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (s + 1 < ns) park((s + 1) & 1);
+        lds_barrier();
+    }
+    const int64_t n = n0 + cbase + jj;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float v = ((acc[0][r] + acc[4][r]) + (acc[2][r] + acc[6][r])) + ((acc[1][r] + acc[5][r]) + (acc[3][r] + acc[7][r]));
+        const int rr = rbase + 4 * q + r;
+        if (rr < rows && n < a.n) a.y[(int64_t)(row0 + rr) * a.ldy + n] = v;
+    }
+}
+
+constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+}  // namespace
+
+// From 9 rows, where no GEMV takes the call or the GEMV would be slower: a
+// GEMV's time grows with the weight bytes it decodes again for every 8 rows
+// (about 0.55 us a MB), the tile's with the blocks of a row while its
+// workgroups are few (0.27 us a block: the chain of one 16 x 16 tile).
+// Measured, tile / GEMV: [8192 x 2048] at 9 / 16 rows 21.6 / 20.8 and 21.6 /
+// 27.1 us, [12288 x 2048] at 9 rows 22 / 32, [4096 x 4096] at 16 rows 37 / 28,
+// [8192 x 4096] at 16 rows 40 / 43, [512 x 2048] at 63 rows 20 / 12, [2048 x
+// 1024] at 63 rows 13 / 16.
+bool q8_tile_supported(const WeightView& w, int64_t m) {
+    if (w.dtype != kQ8_0 || m < 9 || m > (int64_t)1 << 20 || w.rows < 1 || w.cols % (32 * kQtCB) != 0 ||
+        ((uintptr_t)w.w & 3) != 0)
+        return false;
+    return !gemv_supported(w, m) || (double)(w.rows * w.row_bytes) * (double)m / 8 > 1e6 * (0.4 * (double)(w.cols / 32) - 4);
+}
+
+hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
+                          hipStream_t s) {
+    if (!q8_tile_supported(w, m)) return hipErrorNotSupported;
+    QtArgs a;
+    a.w = w.w;
+    a.n = w.rows;
+    a.row_bytes = w.row_bytes;
+    a.nb = (int)(w.cols / 32);
+    a.q = (const int8_t*)ws;
+    a.d = (const float*)((uint8_t*)ws + align256((size_t)(m * w.cols)));
+    a.m = (int)m;
+    a.y = y;
+    a.ldy = ldy;
+    const int64_t qwaves = m * ((w.cols + 255) / 256);
+    hipLaunchKernelGGL(k_qt_quant, dim3((unsigned)((qwaves + 3) / 4)), dim3(256), 0, s, x, ldx, m, w.cols, (int8_t*)a.q,
+                       (float*)a.d);
+    if (hipError_t e = hipGetLastError()) return e;
+    hipLaunchKernelGGL(k_qt_mm, dim3((unsigned)((a.n + kQtCols - 1) / kQtCols), (unsigned)((m + kQtRows - 1) / kQtRows)),
+                       dim3(512), 0, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace iq

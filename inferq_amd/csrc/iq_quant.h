@@ -113,6 +113,25 @@ __device__ __forceinline__ f32x4 q80_vals4_load(const float* xrow, int64_t k, in
     return v;
 }
 
+// Q8_0 of the 8 blocks a wave holds, four values per lane (block l / 8):
+// the lane's int8 packed in a dword and its block's f16 scale.
+struct Q80Lane {
+    uint32_t packed;
+    uint16_t dh;
+};
+__device__ __forceinline__ Q80Lane quant_q80_core(const f32x4 v) {
+    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
+    am = fmaxf(am, __shfl_xor(am, 1));
+    am = fmaxf(am, __shfl_xor(am, 2));
+    am = fmaxf(am, __shfl_xor(am, 4));
+    const float d = __fdiv_rn(am, 127.f);
+    const float id = d != 0.f ? __fdiv_rn(1.f, d) : 0.f;
+    int q[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) q[j] = sat_i8(roundf(v[j] * id));
+    return Q80Lane{pack4(q[0], q[1], q[2], q[3]), f32_to_f16_rne(d)};
+}
+
 // Q8_0 of the 8 blocks of group g of a row of width k (values from
 // q80_vals4_load); `ref_row`, when not null, receives the row's reference
 // 34-byte blocks.
@@ -123,17 +142,9 @@ __device__ __forceinline__ void quant_q80_vals4(const f32x4 v, int64_t k, int64_
     const int64_t nb32 = k / 32;
     const int64_t b = (int64_t)g * 8 + c;  // this lane's Q8_0 block
     const bool valid = b < nb32;
-    float am = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-    am = fmaxf(am, __shfl_xor(am, 1));
-    am = fmaxf(am, __shfl_xor(am, 2));
-    am = fmaxf(am, __shfl_xor(am, 4));
-    const float d = __fdiv_rn(am, 127.f);
-    const float id = d != 0.f ? __fdiv_rn(1.f, d) : 0.f;
-    int q[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) q[j] = sat_i8(roundf(v[j] * id));
-    const uint32_t packed = pack4(q[0], q[1], q[2], q[3]);
-    const uint16_t dh = f32_to_f16_rne(d);
+    const Q80Lane r = quant_q80_core(v);
+    const uint32_t packed = r.packed;
+    const uint16_t dh = r.dh;
     uint32_t* qrow = (uint32_t*)(a.q + row * a.ldq + (int64_t)g * 256);
     qrow[perm_dword(c, kk)] = packed;  // padding lanes store zeros
     if (valid && kk == 0) a.d[row * a.ldd + b] = f16_to_f32(dh);

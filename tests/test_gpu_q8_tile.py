@@ -1,0 +1,72 @@
+"""Q8_0 products at many input rows (iq_q8_tile.hip: the reference's eight
+chains on f16 MFMA), bitwise to the oracle at the edges of its 32 x 64 tiles
+and 4-block stages, and to the lane kernel on rows with no finite scale."""
+import numpy as np
+import pytest
+
+from conftest import assert_bitexact, bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _mat(rows, cols, rng):
+    from inferq_amd import qgemm as Q, synth as S
+
+    w = S.random_matrix(S.Q8_0, rows, cols, rng)
+    return w, Q.QuantizedMatrix.upload(w, S.Q8_0, rows, cols)
+
+
+# widths of 1, 3 and 5 stages of 128 that no GEMV takes (9..63 rows stay on the tile), and whole model widths
+@pytest.mark.parametrize("rows,cols", [(1, 128), (63, 384), (64, 640), (65, 384), (130, 128), (512, 2048), (200, 4096)])
+@pytest.mark.parametrize("m", [9, 16, 17, 31, 32, 33, 64, 97])
+def test_tile_edges_bitwise(gpu, oracle, rows, cols, m):
+    import torch
+
+    from inferq_amd import synth as S
+
+    rng = np.random.default_rng([rows, cols, m])
+    w, mat = _mat(rows, cols, rng)
+    x = S.normal((m, cols), rng)
+    x[0] = 0.0
+    x[m - 1] *= np.float32(1e-20)
+    got = mat.forward(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert_bitexact(got, oracle.matmul(S.Q8_0, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
+
+
+@pytest.mark.parametrize("fill", [0x80, 0x7F, 0xFF, 0x00])
+def test_extreme_values_bitwise(gpu, oracle, fill):
+    """Every weight byte -128, 127, -1 or 0 against rows that quantise to +-127."""
+    import torch
+
+    from inferq_amd import qgemm as Q, synth as S
+
+    rows, cols, m = 70, 640, 40
+    rng = np.random.default_rng(fill)
+    w = S.random_matrix(S.Q8_0, rows, cols, rng).reshape(-1, 34)
+    w[:, 2:] = fill
+    x = np.where(rng.random((m, cols)) < 0.5, np.float32(-3), np.float32(3)).astype(np.float32)
+    x[0], x[1] = 3.0, -3.0
+    mat = Q.QuantizedMatrix.upload(w.reshape(-1), S.Q8_0, rows, cols)
+    got = mat.forward(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert_bitexact(got, oracle.matmul(S.Q8_0, w.reshape(-1), rows, cols, x), f"bytes {fill:#x}")
+
+
+def test_nonfinite_scales_as_the_lane_kernel(gpu):
+    """Infinities and NaN in rows and in weight scales: NaN where the lane kernel has NaN, its bits elsewhere."""
+    import torch
+
+    from inferq_amd import _lib, qgemm as Q, synth as S
+
+    rows, cols, m = 66, 384, 35
+    rng = np.random.default_rng(5)
+    w = S.random_matrix(S.Q8_0, rows, cols, rng).reshape(rows, -1, 34)
+    w[3, 2, 0:2] = np.array([0x7C00], np.uint16).view(np.uint8)  # inf
+    w[7, 0, 0:2] = np.array([0x7E00], np.uint16).view(np.uint8)  # NaN
+    x = S.normal((m, cols), rng)
+    x[2, 5], x[4, 100], x[6, 200] = np.inf, -np.inf, np.nan
+    mat = Q.QuantizedMatrix.upload(w.reshape(-1), S.Q8_0, rows, cols)
+    xd = torch.from_numpy(x).to(gpu)
+    got, ref = (mat.forward_via(xd, p).cpu().numpy() for p in (_lib.PATH_AUTO, _lib.PATH_LANES))
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    assert np.array_equal(bits(got)[ok], bits(ref)[ok])
