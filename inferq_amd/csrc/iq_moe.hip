@@ -709,54 +709,6 @@ hipError_t launch_moe1_g(const MoeParams& p, int dfmt, hipStream_t s, hipEvent_t
     }
 }
 
-// ---------------------------------------------------------------- router
-// Grid (E, ceil(M / TT)), one wave per workgroup: expert e = blockIdx.x
-// against tokens blockIdx.y * TT ..; each lane keeps one partial sum per
-// token over h = lane + 64 j (the router row is read once per TT tokens).
-// U values per lane are loaded before any is summed (one token: U = 32, the
-// whole 2048-wide row in one round trip instead of four), in the same order.
-template <int TT, int U>
-__global__ __launch_bounds__(64) void k_moe_router(MoeParams p) {
-    const int lane = threadIdx.x;
-    const int e = blockIdx.x, t0 = blockIdx.y * TT;
-    const int nt = min(TT, p.M - t0);
-    const int64_t H = p.H;
-    const float* r = p.router + (int64_t)e * H;
-    float part[TT];
-#pragma unroll
-    for (int i = 0; i < TT; i++) part[i] = 0.f;
-    int64_t h = lane;
-    for (; h + 64 * (U - 1) < H; h += 64 * U) {
-        float rv[U];
-#pragma unroll
-        for (int j = 0; j < U; j++) rv[j] = r[h + 64 * j];
-#pragma unroll
-        for (int i = 0; i < TT; i++) {
-            if (i < nt) {
-                const float* xr = p.x + (int64_t)(t0 + i) * H + h;
-                float xv[U];
-#pragma unroll
-                for (int j = 0; j < U; j++) xv[j] = xr[64 * j];
-#pragma unroll
-                for (int j = 0; j < U; j++) part[i] = part[i] + xv[j] * rv[j];
-            }
-        }
-    }
-    for (; h < H; h += 64) {
-        const float rv = r[h];
-#pragma unroll
-        for (int i = 0; i < TT; i++)
-            if (i < nt) part[i] = part[i] + p.x[(int64_t)(t0 + i) * H + h] * rv;
-    }
-#pragma unroll
-    for (int i = 0; i < TT; i++) {
-        float v = part[i];
-#pragma unroll
-        for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off);
-        if (lane == 0 && i < nt) p.logits_ws[(int64_t)(t0 + i) * p.E + e] = v;
-    }
-}
-
 // ------------------------------------------------------------- launchers
 template <int GFMT, int DFMT>
 hipError_t launch_gd(const MoeParams& p, hipStream_t s, hipEvent_t const* ev) {
@@ -878,9 +830,13 @@ hipError_t launch_moe_shared_combine(const float* x, const float* selector, cons
 
 hipError_t launch_moe_router(const MoeParams& p, hipStream_t s) {
     if (!p.router || !p.logits_ws || p.M < 1) return hipErrorInvalidValue;
-    if (p.M <= 2) hipLaunchKernelGGL((k_moe_router<1, 32>), dim3((unsigned)p.E, (unsigned)p.M), dim3(64), 0, s, p);
-    else hipLaunchKernelGGL((k_moe_router<8, 8>), dim3((unsigned)p.E, (unsigned)((p.M + 7) / 8)), dim3(64), 0, s, p);
-    return hipGetLastError();
+    WeightView r;  // the same order as an F32 matrix product
+    r.w = (const uint8_t*)p.router;
+    r.dtype = kF32;
+    r.rows = p.E;
+    r.cols = p.H;
+    r.row_bytes = p.H * 4;
+    return launch_float_mm(r, p.x, p.H, p.M, p.logits_ws, p.E, s);
 }
 
 hipError_t launch_moe_stage(const MoeParams& p, int gfmt, int dfmt, int stage, hipStream_t s) {
