@@ -1,16 +1,19 @@
-// iq_dense_mfma.hip -- y = x . W^T for Q4_K / Q6_K weights at 2..63 input
-// rows on large matrices (the LM head at verify widths), on int8 MFMA in the
-// reference's exact per-lane order (iq_mfma_lanes.h): every output is
-// bitwise what the one-row kernel gives, as src/gguf.rs:493-520 requires of
-// its row tiles.  The per-lane GEMV (iq_gemv.hip) spends eight exact dot
-// chains of VALU work per weight at 8 rows; here the integer dots run on
-// MFMA and the VALU keeps only the f32 chains.
+// iq_dense_mfma.hip -- y = x . W^T for K-quant weights at several input rows,
+// on MFMA in the reference's exact per-lane order: every output is bitwise
+// what the one-row kernel gives, as src/gguf.rs:493-520 requires of its row
+// tiles.  The per-lane GEMV (iq_gemv.hip) spends eight exact dot chains of
+// VALU work per weight at 8 rows; here the integer dots run on MFMA and the
+// VALU keeps only the f32 chains.
 //
-// Two launches per call: k_dm_quant quantises x (Q8K, the lane-transposed
-// activation layout, block scales, 16-value sums as f16); k_dm_mm<FMT, RT>
-// takes 64 weight rows x 16 RT input rows per workgroup, and k_dm_mm_pk
-// 64 weight rows x up to 8 input rows with two reference lanes per MFMA.
+// Two launches per call, the first quantising x (Q8K).  Up to 8 rows
+// (iq_mfma_lanes.h, int8): k_dm_mm_pk takes 64 weight rows per workgroup with
+// two reference lanes per MFMA, k_dm_sk splits K over the waves.  From 9
+// rows k_dh_mm (iq_mfma_half.h, f16) takes 64 weight rows x 16 or 32 input
+// rows; Q6_K's 16-row tiles are k_dm_mm's, on int8.
+#include <algorithm>
+
 #include "iq_internal.h"
+#include "iq_mfma_half.h"
 #include "iq_mfma_lanes.h"
 #include "iq_quant.h"
 
@@ -49,7 +52,57 @@ __global__ __launch_bounds__(256) void k_dm_quant(const float* __restrict__ x, i
     if ((lane & 3) == 0) hs[(row * nb + b) * 16 + (lane >> 2)] = (_Float16)(float)r.bsum16;
 }
 
-// Grid (n / 64, m / (16 RT)): 64 weight rows x 16 RT input rows.
+// As k_dm_quant, the values as f16 in mh_product's order.
+__global__ __launch_bounds__(256) void k_dh_quant(const float* __restrict__ x, int64_t ldx, int m, int nb,
+                                                  int8_t* __restrict__ q, float* __restrict__ d,
+                                                  _Float16* __restrict__ hs) {
+    const int lane = threadIdx.x & 63;
+    const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (wid >= (int64_t)m * nb) return;  // uniform per wave
+    const int64_t row = wid / nb;
+    const int b = (int)(wid - row * nb);
+    const Q8KLane r = quant_q8k_core(load4(x + row * ldx + (int64_t)b * 256 + 4 * lane));
+    mh_store(q + (row * nb + b) * kMhBlock, lane, r.packed);
+    if (lane == 0) d[row * nb + b] = r.d;
+    if ((lane & 3) == 0) hs[(row * nb + b) * 16 + (lane >> 2)] = (_Float16)(float)r.bsum16;
+}
+
+// Grid (n / 64, m / (16 RT)): 64 weight rows x 16 RT input rows on f16 MFMA
+// (mh_product).
+template <int FMT, int RT>
+__global__ __launch_bounds__(256) void k_dh_mm(DmArgs a) {
+    using L = MhStage<FMT, RT>;
+    __shared__ __align__(16) uint8_t st[2][L::END];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = lane >> 4, jj = lane & 15;
+    const int64_t n0 = (int64_t)blockIdx.x * kMlCols;
+    const int row0 = (int)blockIdx.y * 16 * RT;
+    const int rows = min(16 * RT, a.m - row0);
+    MlOperands op;
+    op.aq = a.q;
+    op.ldq = (int64_t)a.nb * kMhBlock;
+    op.ad = a.d;
+    op.ldd = a.nb;
+    op.hs = a.hs;
+    op.b0 = op.b1 = a.w + n0 * a.row_bytes;  // byte offsets stay within the tile's 64 rows
+    op.bsplit = kMlCols;
+    op.brow_bytes = a.row_bytes;
+    op.nb = a.nb;
+    const int64_t last = a.n - 1 - n0;
+    auto brow = [&](int t) -> int64_t { return t < last ? (int64_t)t : last; };
+    auto arow = [&](int rr) -> int64_t { return row0 + min(rr, rows - 1); };
+    float v[4 * RT];
+    mh_product<FMT, RT>(op, arow, brow, st, v);
+    const int64_t n = n0 + 16 * wave + jj;
+#pragma unroll
+    for (int r = 0; r < 4 * RT; r++) {
+        const int rr = 16 * (r >> 2) + 4 * q + (r & 3);
+        if (rr < rows && n < a.n) a.y[(int64_t)(row0 + rr) * a.ldy + n] = v[r];
+    }
+}
+
+// The same on int8 MFMA, with k_dm_quant's activations.
 template <int FMT, int RT>
 __global__ __launch_bounds__(256) void k_dm_mm(DmArgs a) {
     using L = MlStage<FMT, RT>;
@@ -206,13 +259,24 @@ struct DmPlan {
     size_t total() const { return q_bytes + d_bytes + hs_bytes; }
 };
 
+// The row tiles' activations are f16.
 DmPlan dm_plan(const WeightView& w, int64_t m) {
     const int64_t nb = w.cols / 256;
     DmPlan P;
-    P.q_bytes = align256((size_t)(m * nb * 256));
+    P.q_bytes = align256((size_t)(m * nb * (m > 8 || w.dtype == kQ5_K ? kMhBlock : 256)));
     P.d_bytes = align256((size_t)(m * nb * 4));
     P.hs_bytes = align256((size_t)(m * nb * 32));
     return P;
+}
+
+// Rows of one pass: as many as 16 MiB of workspace hold (3912 of width
+// 2048), the call's rows spread evenly.  A wider call runs pass by pass (rows
+// are independent), so that its workspace does not outgrow what it was with
+// int8 activations.
+int64_t dm_pass_rows(const WeightView& w, int64_t m) {
+    const int64_t per_row = w.cols / 256 * (kMhBlock + 36);
+    const int64_t most = std::max<int64_t>((((int64_t)16 << 20) - 1024) / per_row, 1), passes = (m + most - 1) / most;
+    return (m + passes - 1) / passes;
 }
 
 template <int FMT>
@@ -228,6 +292,13 @@ hipError_t launch_pk(const DmArgs& a, hipStream_t s) {
     const dim3 grid((unsigned)((a.n + kMlCols - 1) / kMlCols));
     if (a.amx_key) hipLaunchKernelGGL((k_dm_mm_pk<FMT, true>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((k_dm_mm_pk<FMT, false>), grid, dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+template <int FMT, int RT>
+hipError_t launch_h(const DmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)((a.n + kMlCols - 1) / kMlCols), (unsigned)((a.m + 16 * RT - 1) / (16 * RT)));
+    hipLaunchKernelGGL((k_dh_mm<FMT, RT>), grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -289,7 +360,7 @@ bool dense_mfma_supported(const WeightView& w, int64_t m) {
 }
 
 size_t dense_mfma_workspace_any(const WeightView& w, int64_t m) {
-    return dm_layout_ok(w) && dm_rows_ok(w, m) ? dm_plan(w, m).total() : 0;
+    return dm_layout_ok(w) && dm_rows_ok(w, m) ? dm_plan(w, dm_pass_rows(w, m)).total() : 0;
 }
 
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
@@ -328,9 +399,14 @@ hipError_t launch_dense_argmax(const WeightView& w, const float* x, int64_t m, f
     return dense_run(w, x, w.cols, m, y, w.rows, ws, keys, vals, s);
 }
 
-static hipError_t dense_run(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                            void* ws, uint64_t* amx_key, float* amx_val, hipStream_t s) {
-    if (!dm_layout_ok(w) || !dm_rows_ok(w, m)) return hipErrorNotSupported;
+template <int FMT>
+static hipError_t dense_tiles(const DmArgs& a, bool rt1, hipStream_t s) {
+    if constexpr (FMT == kQ6_K) return rt1 ? launch_t<FMT, 1>(a, s) : launch_h<FMT, 2>(a, s);
+    else return rt1 ? launch_h<FMT, 1>(a, s) : launch_h<FMT, 2>(a, s);
+}
+
+static hipError_t dense_pass(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
+                             void* ws, uint64_t* amx_key, float* amx_val, hipStream_t s) {
     const DmPlan P = dm_plan(w, m);
     uint8_t* base = (uint8_t*)ws;
     DmArgs a;
@@ -346,28 +422,42 @@ static hipError_t dense_run(const WeightView& w, const float* x, int64_t ldx, in
     a.ldy = ldy;
     a.amx_key = amx_key;
     a.amx_val = amx_val;
-    const int64_t qwaves = m * a.nb;
-    hipLaunchKernelGGL(k_dm_quant, dim3((unsigned)((qwaves + 3) / 4)), dim3(256), 0, s, x, ldx, (int)m, a.nb,
-                       (int8_t*)a.q, (float*)a.d, (_Float16*)a.hs);
-    if (hipError_t e = hipGetLastError()) return e;
     // up to 8 rows: the split-K tile on mid-size matrices of width 2048 or 4096
     const bool sk = dm_takes_sk(w, m);
     if (amx_key && (sk || m > 8)) return hipErrorNotSupported;  // fused selection: pair-lane tile only
-    if (w.dtype == kQ5_K && m <= 8) return hipErrorNotSupported;  // Q5_K: row tiles only
     // 16-row tiles up to 16 rows, and wider where 32-row tiles would leave
-    // the GPU short of workgroups (at most 256 of them for Q4_K, 128 for
-    // Q6_K, whose 16-row tiles cost more): [2048 x 4096] Q4_K at 64 / 256
-    // rows 35.4 -> 27.1 / 37.2 -> 30.9 us, [4096 x 2048] Q6_K at 64 rows
-    // 21.7 -> 18.2 us; from 512 workgroups the 32-row tiles win (Q6_K
-    // [8192 x 2048] at 256 rows 45.4 against 59.5 us)
+    // the GPU short of workgroups (16- / 32-row tiles, us: Q4_K [512 x 2048]
+    // at 512 rows, 128 workgroups of 32 rows, 14.8 / 17.5; [2048 x 4096] at
+    // 256 rows, 256 of them, 25.2 / 26.0; [8192 x 2048] at 256 rows, 1024,
+    // 38 / 32; Q5_K [2048 x 4096] at 200 rows, 224, 28.8 / 28.0; Q6_K [2048 x
+    // 4096] at 64 rows, 64, 26 / 29).  Q6_K's 16-row tiles stay on int8 MFMA
+    // (the LM head at 16 rows 115 us, 123 on f16).
     const int64_t g32 = (w.rows + kMlCols - 1) / kMlCols * ((m + 31) / 32);
-    const bool rt1 = m <= 16 || g32 <= (w.dtype == kQ6_K ? 128 : 256);
-    if (w.dtype == kQ5_K) return rt1 ? launch_t<kQ5_K, 1>(a, s) : launch_t<kQ5_K, 2>(a, s);
+    const bool rt1 = m <= 16 || g32 <= (w.dtype == kQ4_K ? 256 : w.dtype == kQ5_K ? 192 : 128);
+    const bool half = w.dtype == kQ5_K || (m > 8 && !(w.dtype == kQ6_K && rt1));
+    const dim3 qgrid((unsigned)((m * a.nb + 3) / 4));
+    if (half)
+        hipLaunchKernelGGL(k_dh_quant, qgrid, dim3(256), 0, s, x, ldx, (int)m, a.nb, (int8_t*)a.q, (float*)a.d,
+                           (_Float16*)a.hs);
+    else
+        hipLaunchKernelGGL(k_dm_quant, qgrid, dim3(256), 0, s, x, ldx, (int)m, a.nb, (int8_t*)a.q, (float*)a.d,
+                           (_Float16*)a.hs);
+    if (hipError_t e = hipGetLastError()) return e;
+    if (w.dtype == kQ5_K) return dense_tiles<kQ5_K>(a, rt1, s);
     if (w.dtype == kQ4_K)
-        return sk ? launch_sk<kQ4_K>(a, s) : m <= 8 ? launch_pk<kQ4_K>(a, s)
-                                       : rt1 ? launch_t<kQ4_K, 1>(a, s) : launch_t<kQ4_K, 2>(a, s);
-    return sk ? launch_sk<kQ6_K>(a, s) : m <= 8 ? launch_pk<kQ6_K>(a, s)
-                                   : rt1 ? launch_t<kQ6_K, 1>(a, s) : launch_t<kQ6_K, 2>(a, s);
+        return sk ? launch_sk<kQ4_K>(a, s) : m <= 8 ? launch_pk<kQ4_K>(a, s) : dense_tiles<kQ4_K>(a, rt1, s);
+    return sk ? launch_sk<kQ6_K>(a, s) : m <= 8 ? launch_pk<kQ6_K>(a, s) : dense_tiles<kQ6_K>(a, rt1, s);
+}
+
+static hipError_t dense_run(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
+                            void* ws, uint64_t* amx_key, float* amx_val, hipStream_t s) {
+    if (!dm_layout_ok(w) || !dm_rows_ok(w, m)) return hipErrorNotSupported;
+    if (w.dtype == kQ5_K && m <= 8) return hipErrorNotSupported;  // a call, not a pass: the GEMV takes those
+    const int64_t pass = dm_pass_rows(w, m);
+    for (int64_t r = 0; r < m; r += pass)
+        if (hipError_t e = dense_pass(w, x + r * ldx, ldx, std::min(pass, m - r), y + r * ldy, ldy, ws, amx_key, amx_val, s))
+            return e;
+    return hipSuccess;
 }
 
 }  // namespace iq

@@ -154,6 +154,17 @@ __device__ __forceinline__ void ml_lds_span(const uint8_t* row, MlShift<S>, int 
     }
 }
 
+// Park 16 staged weight bytes.  The chunks of Q4_K and Q5_K blocks and all but
+// the last of a Q6_K window lie 16-byte aligned in LDS: one 16-byte store,
+// where a dword-aligned vector would go out as two pairs of dwords (exact
+// f16 tile, [512 x 2048] -> 8192 Q4_K: 62 -> 59 us).  The last Q6_K chunk, bytes
+// 196 .. 211 of the window, brings only bytes 208 .. 211 that are not there.
+template <int FMT>
+__device__ __forceinline__ void ml_park_b(uint8_t* dst, const u32x4& v, bool last) {
+    if (FMT == kQ6_K && last) *(uint32_t*)(dst + 12) = v.w;
+    else *(u32x4a16*)dst = u32x4a16{v.x, v.y, v.z, v.w};
+}
+
 // Operands of one tile.  Activation row rr (0 .. 16 RT - 1) of the tile is
 // row arow(rr) of aq (Q8K in the lane-transposed layout, ldq bytes a row),
 // ad (block scales, ldd a row) and hs ([row][nb][16] f16 16-value sums,
@@ -211,13 +222,14 @@ __device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow
     // bytes before the block) as 13 chunks plus one ending at its last byte.
     uint32_t b_src[kBPer];
     int b_off[kBPer];
-    bool b_hi[kBPer];
+    bool b_hi[kBPer], b_last[kBPer];
 #pragma unroll
     for (int i = 0; i < kBPer; i++) {
         const int t = min((int)threadIdx.x + 256 * i, kB - 1);
         const int c2 = t / F::NL, part = t - c2 * F::NL;
         const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
         b_hi[i] = c2 >= op.bsplit;
+        b_last[i] = part == F::NL - 1;
         b_src[i] = (uint32_t)(brow(c2) * op.brow_bytes + po);
         b_off[i] = (int)threadIdx.x + 256 * i < kB ? L::B + c2 * F::BS + po : -1;
     }
@@ -248,7 +260,7 @@ __device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow
             if (a_off[i] >= 0) *(v4i_ml*)(s + a_off[i]) = sa[i];
 #pragma unroll
         for (int i = 0; i < kBPer; i++)
-            if (b_off[i] >= 0) *(u32x4*)(s + b_off[i]) = sb[i];
+            if (b_off[i] >= 0) ml_park_b<FMT>(s + b_off[i], sb[i], b_last[i]);
         if (tD < L::R) *(float*)(s + L::D + 4 * tD) = sd;
         if constexpr (F::kMins)
             if (tH >= 0 && tH < 2 * L::R) *(v4i_ml*)(s + L::H + 32 * (tH >> 1) + 16 * (tH & 1)) = sh16;
@@ -628,13 +640,14 @@ __device__ __forceinline__ void ml_product_pk(const MlOperands& op, ARow arow, B
     const int a_off = ta < kA ? L::A + (ta >> 4) * kMlAS + 16 * (ta & 15) : -1;
     uint32_t b_src[kBPer];
     int b_off[kBPer];
-    bool b_hi[kBPer];
+    bool b_hi[kBPer], b_last[kBPer];
 #pragma unroll
     for (int i = 0; i < kBPer; i++) {
         const int t = min((int)threadIdx.x + 256 * i, kB - 1);
         const int c2 = t / F::NL, part = t - c2 * F::NL;
         const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
         b_hi[i] = c2 >= op.bsplit;
+        b_last[i] = part == F::NL - 1;
         b_src[i] = (uint32_t)(brow(c2) * op.brow_bytes + po);
         b_off[i] = (int)threadIdx.x + 256 * i < kB ? L::B + c2 * F::BS + po : -1;
     }
@@ -660,7 +673,7 @@ __device__ __forceinline__ void ml_product_pk(const MlOperands& op, ARow arow, B
         if (a_off >= 0) *(v4i_ml*)(s + a_off) = sa;
 #pragma unroll
         for (int i = 0; i < kBPer; i++)
-            if (b_off[i] >= 0) *(u32x4*)(s + b_off[i]) = sb[i];
+            if (b_off[i] >= 0) ml_park_b<FMT>(s + b_off[i], sb[i], b_last[i]);
         if (tD >= 0 && tD < 8) *(float*)(s + L::D + 4 * tD) = sd;
         if constexpr (F::kMins)
             if (tH >= 0 && tH < 16) *(v4i_ml*)(s + L::H + 32 * (tH >> 1) + 16 * (tH & 1)) = sh16;
@@ -775,7 +788,7 @@ __device__ __forceinline__ void ml_product_sk(const MlOperands& op, ARow arow, B
         if (t < kB) {
             const int cb = t / F::NL, part = t - cb * F::NL, col = cb / BPW, bi = cb - col * BPW;
             const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
-            *(u32x4*)(reg[wave][bi] + R::B + col * F::BS + po) = sb[i];
+            ml_park_b<FMT>(reg[wave][bi] + R::B + col * F::BS + po, sb[i], part == F::NL - 1);
         }
     }
     if (lane < 8 * BPW) *(float*)(reg[wave][lane >> 3] + R::D + 4 * (lane & 7)) = sd;
@@ -985,13 +998,14 @@ __device__ __forceinline__ void ml_product_tiles(const MlOperands& op, ARow arow
     }
     uint32_t b_src[kBPer];
     int b_off[kBPer];
-    bool b_hi[kBPer];
+    bool b_hi[kBPer], b_last[kBPer];
 #pragma unroll
     for (int i = 0; i < kBPer; i++) {
         const int t = min((int)threadIdx.x + 256 * i, kB - 1);
         const int c2 = t / F::NL, part = t - c2 * F::NL;
         const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
         b_hi[i] = c2 >= op.bsplit;
+        b_last[i] = part == F::NL - 1;
         b_src[i] = (uint32_t)(brow(c2) * op.brow_bytes + po);
         b_off[i] = (int)threadIdx.x + 256 * i < kB ? L::B + c2 * F::BS + po : -1;
     }
@@ -1021,7 +1035,7 @@ __device__ __forceinline__ void ml_product_tiles(const MlOperands& op, ARow arow
             if (a_off[i] >= 0) *(v4i_ml*)(s + a_off[i]) = sa[i];
 #pragma unroll
         for (int i = 0; i < kBPer; i++)
-            if (b_off[i] >= 0) *(u32x4*)(s + b_off[i]) = sb[i];
+            if (b_off[i] >= 0) ml_park_b<FMT>(s + b_off[i], sb[i], b_last[i]);
         if (tD < L::R) *(float*)(s + L::D + 4 * tD) = sd;
         if constexpr (F::kMins)
             if (tH >= 0 && tH < 2 * L::R) *(v4i_ml*)(s + L::H + 32 * (tH >> 1) + 16 * (tH & 1)) = sh16;

@@ -485,11 +485,13 @@ __device__ __forceinline__ void mp_down_res_body(const MoeParams& p, const MpChu
     constexpr int kB = kMlCols * F::NL, kBPer = (kB + 255) / 256;
     uint32_t b_src[kBPer];
     int b_off[kBPer];
+    bool b_last[kBPer];
 #pragma unroll
     for (int i = 0; i < kBPer; i++) {
         const int t = min((int)threadIdx.x + 256 * i, kB - 1);
         const int c2 = t / F::NL, part = t - c2 * F::NL;
         const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
+        b_last[i] = part == F::NL - 1;
         b_src[i] = (uint32_t)(c2 * p.d_row_bytes + po);
         b_off[i] = (int)threadIdx.x + 256 * i < kB ? c2 * F::BS + po : -1;
     }
@@ -506,7 +508,7 @@ __device__ __forceinline__ void mp_down_res_body(const MoeParams& p, const MpChu
         uint8_t* st = lds + Lr::B + (s & 1) * Lr::BST;
 #pragma unroll
         for (int i = 0; i < kBPer; i++)
-            if (b_off[i] >= 0) *(u32x4*)(st + b_off[i]) = sb[s & 1][i];
+            if (b_off[i] >= 0) ml_park_b<FMT>(st + b_off[i], sb[s & 1][i], b_last[i]);
     };
     constexpr int NS = NCT * NB;
     // ---- the chunk's activations, once: NB blocks x 16 NT rows x 16

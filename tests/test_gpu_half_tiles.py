@@ -1,0 +1,62 @@
+"""K-quant products on the f16 MFMA row tiles (iq_mfma_half.h), bitwise to the
+oracle at the edges of their 16 / 32 x 64 tiles, on blocks of extreme bytes,
+and across the passes of a call wider than one pass's workspace."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import assert_bitexact
+from inferq_amd import qgemm as Q
+from inferq_amd import synth as S
+
+pytestmark = pytest.mark.gpu
+
+
+# few weight rows run on 16-row tiles, many (or wide calls) on 32-row tiles
+@pytest.mark.parametrize("rows,cols,m", [(1, 256, 64), (63, 512, 65), (65, 768, 79), (130, 256, 97), (8256, 512, 64),
+                                         (8200, 256, 95), (4100, 512, 161)])
+@pytest.mark.parametrize("dtype", [S.Q4_K, S.Q5_K, S.Q6_K])
+def test_tile_edges_bitwise(gpu, oracle, dtype, rows, cols, m):
+    if dtype == S.Q6_K and cols % 512:
+        cols *= 2  # an even block count keeps rows dword-aligned
+    rng = np.random.default_rng([dtype, rows, cols, m])
+    w = S.random_matrix(dtype, rows, cols, rng)
+    x = S.normal((m, cols), rng)
+    x[0] = 0.0
+    got = Q.QuantizedMatrix.upload(w, dtype, rows, cols).forward(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert_bitexact(got, oracle.matmul(dtype, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
+
+
+@pytest.mark.parametrize("fill", [0xFF, 0x80, 0x7F, 0x00])
+@pytest.mark.parametrize("dtype", [S.Q4_K, S.Q5_K, S.Q6_K])
+def test_extreme_integers_bitwise(gpu, oracle, dtype, fill):
+    """Every payload byte at an extreme (scales 63, -1, -128, 127; quants 0 or largest) against rows of +-128."""
+    rows, cols, m = 8256, 512, 70
+    w = S.random_matrix(dtype, rows, cols, np.random.default_rng(fill)).reshape(-1, S.BLOCK_BYTES[dtype])
+    w[:, (slice(0, 208) if dtype == S.Q6_K else slice(4, None))] = fill
+    x = np.full((m, cols), -3.0, np.float32)
+    x[1::3] = 3.0
+    x[2::3, ::2] = 3.0
+    got = Q.QuantizedMatrix.upload(w.reshape(-1), dtype, rows, cols).forward(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert_bitexact(got, oracle.matmul(dtype, w.reshape(-1), rows, cols, x), f"bytes {fill:#x}")
+
+
+@pytest.mark.parametrize("dtype", [S.Q4_K, S.Q5_K, S.Q6_K])
+def test_passes_match_narrow_calls(gpu, dtype):
+    """A call past one pass (16 MiB of f16 activations) gives each row what a call of 64 rows gives it, also through
+    the allocation-free entry, whose 16 MiB it must not outgrow."""
+    from inferq_amd._lib import check, lib
+
+    rows, cols, m = 40, 8192, 1100  # 957 rows a pass
+    rng = np.random.default_rng(dtype)
+    mat = Q.QuantizedMatrix.upload(S.random_matrix(dtype, rows, cols, rng), dtype, rows, cols)
+    x = torch.from_numpy(S.normal((m, cols), rng)).to(gpu)
+    got = mat.forward(x)
+    want = torch.cat([mat.forward(x[i:i + 64].contiguous()) for i in range(0, 1024, 64)] +
+                     [mat.forward(x[1024:].contiguous())])
+    assert torch.equal(got.view(torch.int32), want.view(torch.int32))
+    y = torch.empty_like(got)
+    torch.cuda.synchronize()
+    check(lib().iq_matmul_noalloc(mat.handle, x.data_ptr(), m, y.data_ptr(), None))
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int32), got.view(torch.int32))
