@@ -52,6 +52,8 @@ struct MoeParams {
     // MFMA (prefill) path
     _Float16* xhs = nullptr;        // [M][H/256][16] 16-value sums of quantised x
     _Float16* ahs = nullptr;        // [P][I/256][16] the same of quantised act
+    int8_t* xh = nullptr;           // [M][H/256][512] quantised x as f16 (iq_mfma_half.h), for Q4_K / Q5_K gate and up
+    int8_t* ah = nullptr;           // [P][I/256][512] quantised act as f16, for Q4_K / Q5_K down
     int32_t* chunk_group = nullptr;  // [max_chunks] group of each chunk of rows
     int32_t* chunk_r0 = nullptr;     // [max_chunks] first row of the chunk in its group
     int max_chunks = 0;

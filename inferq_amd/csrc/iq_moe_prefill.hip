@@ -27,6 +27,7 @@
 #include <type_traits>
 
 #include "iq_lanes.h"
+#include "iq_mfma_half.h"
 #include "iq_mfma_lanes.h"
 #include "iq_moe.h"
 #include "iq_quant.h"
@@ -50,6 +51,12 @@ constexpr int kMpRouteTok = 4;
 // ones cost in repeated weight decode (the call: 184 -> 167 us).
 constexpr int kMpRT = 1;  // 16-row MFMA tiles per chunk
 static_assert(kMpRows == 16 * kMpRT, "chunk rows");
+// Expert products of a format that run on f16 MFMA (mh_product): the gate/up
+// launch of 256 tokens, Dirichlet routing, Q4_K, 78 -> 66 us, the Q5_K down
+// launch of 512 tokens 78 -> 70.  Q6_K keeps the
+// int8 tiles, which at 16 rows decode it faster.
+template <int FMT>
+constexpr bool kMpHalf = FMT == kQ4_K || FMT == kQ5_K;
 constexpr int kMpTileRT = kMpTileRows / 16;  // 16-row tiles per chunk of the tile-order down
 #ifndef IQ_MP_RES_CT
 #define IQ_MP_RES_CT 2
@@ -62,6 +69,7 @@ constexpr int kMpTileRT = kMpTileRows / 16;  // 16-row tiles per chunk of the ti
 constexpr int kMpResCT = IQ_MP_RES_CT;
 
 // ------------------------------------------------------------ routing
+template <bool HALF>
 __global__ __launch_bounds__(kMpThreads) void k_mp_route(MoeParams p) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -114,7 +122,8 @@ __global__ __launch_bounds__(kMpThreads) void k_mp_route(MoeParams p) {
     const int64_t row = wid / nb;
     const int b = (int)(wid - row * nb);
     const Q8KLane r = quant_q8k_core(load4(p.x + row * p.H + (int64_t)b * 256 + 4 * lane));
-    ((uint32_t*)(p.xq.q + row * p.xq.ldq + (int64_t)b * 256))[perm_dword(lane >> 3, lane & 7)] = r.packed;
+    if constexpr (HALF) mh_store(p.xh + (row * nb + b) * kMhBlock, lane, r.packed);
+    else ((uint32_t*)(p.xq.q + row * p.xq.ldq + (int64_t)b * 256))[perm_dword(lane >> 3, lane & 7)] = r.packed;
     if (lane == 0) p.xq.d[row * p.xq.ldd + b] = r.d;
     if ((lane & 3) == 0) p.xhs[(row * nb + b) * 16 + (lane >> 2)] = (_Float16)(float)r.bsum16;
 }
@@ -286,12 +295,12 @@ __global__ __launch_bounds__(kMpThreads) void k_mp_group(MoeParams p) {
 // results into vals.
 template <int FMT, int MODE>
 __global__ __launch_bounds__(256) void k_mp_mm(MoeParams p) {
-    using L = MlStage<FMT, kMpRT>;
+    constexpr bool HALF = kMpHalf<FMT>;
+    using L = std::conditional_t<HALF, MhStage<FMT, kMpRT>, MlStage<FMT, kMpRT>>;
     using LP = MlStagePk<FMT>;
-    constexpr int kStage = 2 * L::END > 2 * LP::END ? 2 * L::END : 2 * LP::END;
-    __shared__ __align__(16) uint8_t lds[kStage + 256];
+    constexpr int kStage = HALF || 2 * L::END > 2 * LP::END ? 2 * L::END : 2 * LP::END;
+    __shared__ __align__(16) uint8_t lds[kStage + (HALF ? 0 : 256)];
     auto st = (uint8_t (*)[L::END])lds;
-    uint8_t* zero = lds + kStage;
     const int c = blockIdx.y;
     if (c >= p.meta[1]) return;  // whole workgroup
     const int lane = threadIdx.x & 63;
@@ -305,12 +314,12 @@ __global__ __launch_bounds__(256) void k_mp_mm(MoeParams p) {
 
     MlOperands op;
     const ActView& av = MODE == 0 ? p.xq : p.aq;
-    op.aq = av.q;
-    op.ldq = av.ldq;
+    op.nb = MODE == 0 ? p.g_nbw : p.d_nbw;  // weight blocks per row = activation blocks
+    op.aq = !HALF ? av.q : MODE == 0 ? p.xh : p.ah;
+    op.ldq = HALF ? (int64_t)op.nb * kMhBlock : av.ldq;
     op.ad = av.d;
     op.ldd = av.ldd;
     op.hs = MODE == 0 ? p.xhs : p.ahs;
-    op.nb = MODE == 0 ? p.g_nbw : p.d_nbw;  // weight blocks per row = activation blocks
     op.brow_bytes = MODE == 0 ? p.g_row_bytes : p.d_row_bytes;
     if constexpr (MODE == 0) {
         op.b0 = shared ? p.sgate_w : p.gate + (int64_t)e * p.g_exp_bytes;
@@ -334,17 +343,18 @@ __global__ __launch_bounds__(256) void k_mp_mm(MoeParams p) {
     // of a lane is then row 4 (q & 1) + r (every lane group), else row
     // 16 (r / 4) + 4 q + r % 4
     float v[4 * kMpRT];
-    // uniform per workgroup; Q5_K has no pair-lane form and takes the
-    // 16-row tile for every chunk
-    const bool pk = FMT != kQ5_K && rows <= 8;
-    if (pk) {
-        if constexpr (FMT != kQ5_K) {
-            ((uint32_t*)zero)[threadIdx.x & 63] = 0u;  // read only after the product's first barrier
-            float vp[4];
-            ml_product_pk<FMT>(op, arow, brow, (uint8_t (*)[LP::END])lds, zero, vp);
+    // uniform per workgroup; the f16 tile takes chunks of any size (at 8 rows
+    // it costs less than the pair-lane tile, whose decode is the same)
+    const bool pk = !HALF && rows <= 8;
+    if constexpr (HALF) {
+        mh_product<FMT, kMpRT>(op, arow, brow, st, v);
+    } else if (pk) {
+        uint8_t* zero = lds + kStage;
+        ((uint32_t*)zero)[threadIdx.x & 63] = 0u;  // read only after the product's first barrier
+        float vp[4];
+        ml_product_pk<FMT>(op, arow, brow, (uint8_t (*)[LP::END])lds, zero, vp);
 #pragma unroll
-            for (int r = 0; r < 4 * kMpRT; r++) v[r] = r < 4 ? vp[r] : 0.f;
-        }
+        for (int r = 0; r < 4 * kMpRT; r++) v[r] = r < 4 ? vp[r] : 0.f;
     } else {
         ml_product<FMT, kMpRT>(op, arow, brow, st, v);
     }
@@ -612,7 +622,7 @@ __global__ __launch_bounds__(256) void k_mp_down_res(MoeParams p) {
 
 // ------------------------------------------- act quantisation, combine
 // One wave per (grouped row, 256-value block) of act.
-template <int DFMT>
+template <int DFMT, bool HALF>
 __global__ __launch_bounds__(256) void k_mp_actq(MoeParams p, int P) {
     const int lane = threadIdx.x & 63;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -621,7 +631,8 @@ __global__ __launch_bounds__(256) void k_mp_actq(MoeParams p, int P) {
     const int64_t row = wid / nb;
     const int b = (int)(wid - row * nb);
     const Q8KLane r = quant_q8k_core(load4(p.act + row * p.I + (int64_t)b * 256 + 4 * lane));
-    ((uint32_t*)(p.aq.q + row * p.aq.ldq + (int64_t)b * 256))[perm_dword(lane >> 3, lane & 7)] = r.packed;
+    if constexpr (HALF) mh_store(p.ah + (row * nb + b) * kMhBlock, lane, r.packed);
+    else ((uint32_t*)(p.aq.q + row * p.aq.ldq + (int64_t)b * 256))[perm_dword(lane >> 3, lane & 7)] = r.packed;
     if (lane == 0) p.aq.d[row * p.aq.ldd + b] = r.d;
     if constexpr (DFMT == kQ4_K || DFMT == kQ5_K)  // the down products' mins
         if ((lane & 3) == 0) p.ahs[(row * nb + b) * 16 + (lane >> 2)] = (_Float16)(float)r.bsum16;
@@ -682,7 +693,7 @@ hipError_t launch_p(const MoeParams& p, hipStream_t s, hipEvent_t const* ev) {
     if (ev) (void)hipEventRecord(ev[0], s);
     const int nr = (M + kMpRouteTok - 1) / kMpRouteTok;
     const int64_t qw = (int64_t)M * nbH;
-    hipLaunchKernelGGL(k_mp_route, dim3((unsigned)(nr + (qw + 15) / 16)), dim3(kMpThreads), 0, s, p);
+    hipLaunchKernelGGL((k_mp_route<kMpHalf<GFMT>>), dim3((unsigned)(nr + (qw + 15) / 16)), dim3(kMpThreads), 0, s, p);
     if (hipError_t e = hipGetLastError()) return e;
     const size_t mask_bytes = (size_t)p.E * ((M + 31) / 32) * 4;
     hipLaunchKernelGGL(k_mp_group, dim3(1), dim3(kMpThreads), mask_bytes, s, p);
@@ -691,7 +702,11 @@ hipError_t launch_p(const MoeParams& p, hipStream_t s, hipEvent_t const* ev) {
     hipLaunchKernelGGL((k_mp_mm<GFMT, 0>), dim3((unsigned)(p.I / 32), (unsigned)p.max_chunks), dim3(256), 0, s, p);
     if (hipError_t e = hipGetLastError()) return e;
     const int64_t aw = (int64_t)P * p.aq.ng;
-    hipLaunchKernelGGL((k_mp_actq<DFMT>), dim3((unsigned)((aw + 3) / 4)), dim3(256), 0, s, p, P);
+    // the tile-order forms of a Q4_K down read int8
+    if (kMpHalf<DFMT> && !(p.down_tiles && DFMT != kQ5_K))
+        hipLaunchKernelGGL((k_mp_actq<DFMT, true>), dim3((unsigned)((aw + 3) / 4)), dim3(256), 0, s, p, P);
+    else
+        hipLaunchKernelGGL((k_mp_actq<DFMT, false>), dim3((unsigned)((aw + 3) / 4)), dim3(256), 0, s, p, P);
     if (hipError_t e = hipGetLastError()) return e;
     if (ev) (void)hipEventRecord(ev[2], s);
     if constexpr (DFMT == kQ5_K) {  // no tile-order form: the exact products on either path
@@ -730,7 +745,7 @@ bool moep_supported(const MoeParams& p, int gfmt, int dfmt) {
                          al(p.residual, 16);  // k_mp_combine moves four floats at a time
     return kq && aligned && p.M >= kMoePrefillMinTokens && p.H % 256 == 0 && p.I % 256 == 0 && p.E <= kMoeMaxExperts &&
            p.K <= kMoeMaxTopK && p.g_row_bytes % 4 == 0 && p.d_row_bytes % 4 == 0 &&
-           (int64_t)p.E * ((p.M + 31) / 32) * 4 <= 32768 && p.xhs != nullptr && p.chunk_group != nullptr &&
+           (int64_t)p.E * ((p.M + 31) / 32) * 4 <= 32768 && p.xhs != nullptr && p.chunk_group != nullptr && p.xh != nullptr && p.ah != nullptr &&
            ((dfmt != kQ4_K && dfmt != kQ5_K) || p.ahs != nullptr);
 }
 
