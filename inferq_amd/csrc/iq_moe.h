@@ -71,6 +71,11 @@ struct MoeParams {
     int32_t* tchunk_group = nullptr;  // [max_tchunks]
     int32_t* tchunk_r0 = nullptr;     // [max_tchunks]
     int max_tchunks = 0;
+    // the caller's copy of the routes, or null: the kernel that combines a
+    // token's outputs writes it (two copies on the stream cost a one-token
+    // call about 3 of 20 us)
+    int32_t* experts_out = nullptr;  // [M][K]
+    float* weights_out = nullptr;    // [M][K]
 };
 
 constexpr int kMpRows = 16;  // grouped rows per chunk of the exact expert products

@@ -251,6 +251,11 @@ __global__ __launch_bounds__(256) void k_moe_down(MoeParams p) {
     // then hidden = routed + shared * gate (src/qwen/quantized_moe.rs:266-273,
     // :384-400)
     const int K = (int)p.K;
+    if (blockIdx.x == 0)
+        for (int a = threadIdx.x; a < p.M * K; a += 256) {
+            if (p.experts_out) p.experts_out[a] = p.experts[a];
+            if (p.weights_out) p.weights_out[a] = p.weights[a];
+        }
     for (int idx = threadIdx.x; idx < p.M * 8; idx += 256) {
         const int t = idx >> 3;
         const int64_t nn = (int64_t)blockIdx.x * 8 + (idx & 7);
@@ -630,6 +635,10 @@ __global__ __launch_bounds__(1024) void k_moe1_down(MoeParams p) {
     float o[1][1];
     lanes_finish<DFMT, 1, 1>(acc, accm, o);
     if (k == 0) s_vals[wave][slot] = o[0][0];
+    if (blockIdx.x == 0 && lane == 0 && wave < K) {
+        if (p.experts_out) p.experts_out[t * K + wave] = e;
+        if (p.weights_out) p.weights_out[t * K + wave] = p.weights[t * K + wave];
+    }
     __syncthreads();
     if (threadIdx.x < 8) {
         const int64_t nn = (int64_t)blockIdx.x * 8 + threadIdx.x;
@@ -792,24 +801,44 @@ __global__ __launch_bounds__(256) void k_moe_swiglu(const float* __restrict__ g,
 // out[t] = residual[t] + (out[t] + shared[t] * sigmoid(x[t] . selector)):
 // `out` holds the routed sum (the routed launches ran without the shared
 // expert and the residual), so the additions keep the fused kernels' order.
-// Grid (ceil(H / 256), M); wave 0 forms the token's gate.
+// Grid M: wave 0 forms the token's gate while every wave's values are in
+// flight (a workgroup per 256 columns formed it again for each: 512 tokens
+// 11.1 -> 5.8 us).
 __global__ __launch_bounds__(256) void k_moe_shared_combine(const float* __restrict__ x,
                                                             const float* __restrict__ selector,
                                                             const float* __restrict__ shared,
                                                             const float* __restrict__ residual, int64_t H,
                                                             float* __restrict__ out) {
+    constexpr int U = 8;
     __shared__ float s_gate;
-    const int64_t t = blockIdx.y;
-    if (threadIdx.x < 64) {
-        const float gate = selector_gate(x + t * H, selector, H);
-        if (threadIdx.x == 0) s_gate = gate;
+    const int64_t t = blockIdx.x;
+    out += t * H;
+    shared += t * H;
+    if (residual) residual += t * H;
+    for (int64_t n0 = threadIdx.x; n0 - threadIdx.x < H; n0 += 256 * U) {
+        float o[U], sv[U], rv[U];
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int64_t n = min(n0 + 256 * j, H - 1);
+            o[j] = out[n];
+            sv[j] = shared[n];
+            rv[j] = residual ? residual[n] : 0.f;
+        }
+        if (n0 < 256) {  // the first pass, uniform
+            if (threadIdx.x < 64) {
+                const float gate = selector_gate(x + t * H, selector, H);
+                if (threadIdx.x == 0) s_gate = gate;
+            }
+            __syncthreads();
+        }
+#pragma unroll
+        for (int j = 0; j < U; j++) {
+            const int64_t n = n0 + 256 * j;
+            float v = o[j] + sv[j] * s_gate;
+            if (residual) v = rv[j] + v;  // src/qwen/quantized_layer.rs:212
+            if (n < H) out[n] = v;
+        }
     }
-    __syncthreads();
-    const int64_t n = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (n >= H) return;
-    float v = out[t * H + n] + shared[t * H + n] * s_gate;
-    if (residual) v = residual[t * H + n] + v;  // src/qwen/quantized_layer.rs:212
-    out[t * H + n] = v;
 }
 
 
@@ -823,8 +852,7 @@ hipError_t launch_moe_swiglu(const float* g, const float* u, int64_t n, float* a
 hipError_t launch_moe_shared_combine(const float* x, const float* selector, const float* shared, const float* residual,
                                      int64_t m, int64_t H, float* out, hipStream_t s) {
     if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_moe_shared_combine, dim3((unsigned)((H + 255) / 256), (unsigned)m), dim3(256), 0, s, x,
-                       selector, shared, residual, H, out);
+    hipLaunchKernelGGL(k_moe_shared_combine, dim3((unsigned)m), dim3(256), 0, s, x, selector, shared, residual, H, out);
     return hipGetLastError();
 }
 

@@ -306,6 +306,8 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
     p.out = out;
     // a shared expert run apart adds its term and the residual at the end
     p.residual = L->shared_apart ? nullptr : residual;
+    p.experts_out = experts_out;
+    p.weights_out = weights_out;
     L->has_last = false;
     hipError_t e = hipSuccess;
     if (logits) {
@@ -336,12 +338,9 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
         if (e != hipSuccess) return hip_fail(e, "MoE shared combine launch");
     }
     L->last = p;
+    L->last.experts_out = nullptr;  // a stage launched again leaves the routes alone
+    L->last.weights_out = nullptr;
     L->has_last = true;
-    const size_t rb = (size_t)(m * L->layer.K) * 4;
-    if (experts_out && (e = hipMemcpyAsync(experts_out, p.experts, rb, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_fail(e, "hipMemcpyAsync (experts)");
-    if (weights_out && (e = hipMemcpyAsync(weights_out, p.weights, rb, hipMemcpyDeviceToDevice, s)) != hipSuccess)
-        return hip_fail(e, "hipMemcpyAsync (weights)");
     return IQ_OK;
 }
 
