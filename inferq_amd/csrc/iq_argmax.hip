@@ -25,8 +25,17 @@ namespace iq {
 namespace {
 
 constexpr int kArgmaxThreads = 256;
-constexpr int kArgmaxPerThread = 16;
-constexpr int64_t kArgmaxChunk = (int64_t)kArgmaxThreads * kArgmaxPerThread;
+// Logits per thread: four up to 16 rows (243 workgroups a row of 248320
+// logits, where sixteen a thread leave 61, most CUs idle and each thread a
+// long chain of key compares: one row 6.8 -> 4.9 us, eight 7.6 -> 6.1),
+// sixteen for more rows, which fill the GPU by themselves (64 rows 19.6 us,
+// 22.8 with four).
+constexpr int kArgmaxFewRows = 16;
+constexpr int argmax_per_thread(int64_t m) { return m <= kArgmaxFewRows ? 4 : 16; }
+constexpr int64_t argmax_chunks(int64_t m, int64_t n) {
+    const int64_t chunk = (int64_t)kArgmaxThreads * argmax_per_thread(m);
+    return (n + chunk - 1) / chunk;
+}
 
 __device__ __forceinline__ uint64_t max_u64(uint64_t a, uint64_t b) { return a > b ? a : b; }
 
@@ -46,15 +55,16 @@ __device__ __forceinline__ uint64_t block_max(uint64_t key) {
     return key;
 }
 
-// Grid (chunks, m): chunk c of row r covers [c * kArgmaxChunk, ...).
+// Grid (chunks, m): chunk c of row r covers [c * 256 PT, ...).
+template <int PT>
 __global__ __launch_bounds__(kArgmaxThreads) void k_argmax_part(const float* __restrict__ y, int64_t ldy, int64_t n,
                                                                 uint64_t* __restrict__ part, int chunks) {
     const int64_t r = blockIdx.y;
-    const int64_t base = (int64_t)blockIdx.x * kArgmaxChunk;
+    const int64_t base = (int64_t)blockIdx.x * (kArgmaxThreads * PT);
     const float* row = y + r * ldy;
     uint64_t key = 0;
 #pragma unroll
-    for (int j = 0; j < kArgmaxPerThread; j++) {
+    for (int j = 0; j < PT; j++) {
         const int64_t i = base + (int64_t)j * kArgmaxThreads + threadIdx.x;
         if (i < n) key = max_u64(key, argmax_key(row[i], i));
     }
@@ -139,18 +149,21 @@ hipError_t launch_argmax_kv(const uint64_t* keys, const float* vals, int64_t m, 
 }
 
 size_t argmax_workspace_size(int64_t m, int64_t n) {
-    const int64_t chunks = (n + kArgmaxChunk - 1) / kArgmaxChunk;
-    return (size_t)(m * chunks) * sizeof(uint64_t);
+    // what a call of any number of rows up to m needs
+    const int64_t few = m < kArgmaxFewRows ? m : kArgmaxFewRows;
+    const int64_t a = m * argmax_chunks(m, n), b = few * argmax_chunks(few, n);
+    return (size_t)(a > b ? a : b) * sizeof(uint64_t);
 }
 
 hipError_t launch_argmax(const float* y, int64_t m, int64_t n, int64_t ldy, int32_t* idx, float* val, void* ws,
                          hipStream_t s) {
     if (m <= 0 || n <= 0) return hipSuccess;
     if (n > INT32_MAX || m > 65535) return hipErrorInvalidValue;
-    const int chunks = (int)((n + kArgmaxChunk - 1) / kArgmaxChunk);
+    const int chunks = (int)argmax_chunks(m, n);
     uint64_t* part = (uint64_t*)ws;
-    hipLaunchKernelGGL(k_argmax_part, dim3((unsigned)chunks, (unsigned)m), dim3(kArgmaxThreads), 0, s, y, ldy, n,
-                       part, chunks);
+    const dim3 grid((unsigned)chunks, (unsigned)m);
+    if (argmax_per_thread(m) == 4) hipLaunchKernelGGL((k_argmax_part<4>), grid, dim3(kArgmaxThreads), 0, s, y, ldy, n, part, chunks);
+    else hipLaunchKernelGGL((k_argmax_part<16>), grid, dim3(kArgmaxThreads), 0, s, y, ldy, n, part, chunks);
     if (hipError_t e = hipGetLastError()) return e;
     hipLaunchKernelGGL(k_argmax_final, dim3((unsigned)m), dim3(kArgmaxThreads), 0, s, y, ldy, part, chunks, idx, val);
     return hipGetLastError();
