@@ -90,6 +90,12 @@ bool q8_tile_supported(const WeightView& w, int64_t m);
 hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
                           hipStream_t s);
 
+// out[m] = down . SwiGLU(gate . x, up . x) on Q8_0 matrices where
+// q8_tile_supported takes all three (else hipErrorNotSupported, nothing
+// launched); g and u [m][gate.rows], `ws` at least act_bytes of either width.
+hipError_t launch_q8_swiglu(const WeightView& gate, const WeightView& up, const WeightView& down, const float* x,
+                            int64_t m, float* g, float* u, float* out, void* ws, hipStream_t s);
+
 // y[m][ldy] = x . W^T for F32 and BF16 matrices (iq_dense_f32.hip), in the
 // MoE router's f32 order; hipErrorNotSupported for other dtypes.
 hipError_t launch_float_mm(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,

@@ -323,17 +323,22 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
         // the reference's shared path: down(SwiGLU(gate . x, up . x)), then
         // out = residual + (routed + shared * sigmoid(x . selector))
         const int64_t I = L->layer.I, H = L->layer.H;
-        if (int rc = matmul_impl(&L->sgate, x, m, p.shared_g, p.shared_ws, p.shared_ws_bytes, IQ_PATH_AUTO, nullptr,
-                                 nullptr, s))
-            return rc;
-        if (int rc = matmul_impl(&L->sup, x, m, p.shared_u, p.shared_ws, p.shared_ws_bytes, IQ_PATH_AUTO, nullptr,
-                                 nullptr, s))
-            return rc;
-        e = launch_moe_swiglu(p.shared_g, p.shared_u, m * I, p.shared_act, s);
-        if (e != hipSuccess) return hip_fail(e, "MoE shared SwiGLU launch");
-        if (int rc = matmul_impl(&L->sdown, p.shared_act, m, p.shared_out, p.shared_ws, p.shared_ws_bytes,
-                                 IQ_PATH_AUTO, nullptr, nullptr, s))
-            return rc;
+        e = launch_q8_swiglu(view_of(&L->sgate), view_of(&L->sup), view_of(&L->sdown), x, m, p.shared_g, p.shared_u,
+                             p.shared_out, p.shared_ws, s);
+        if (e != hipSuccess && e != hipErrorNotSupported) return hip_fail(e, "MoE shared expert launch");
+        if (e == hipErrorNotSupported) {
+            if (int rc = matmul_impl(&L->sgate, x, m, p.shared_g, p.shared_ws, p.shared_ws_bytes, IQ_PATH_AUTO, nullptr,
+                                     nullptr, s))
+                return rc;
+            if (int rc = matmul_impl(&L->sup, x, m, p.shared_u, p.shared_ws, p.shared_ws_bytes, IQ_PATH_AUTO, nullptr,
+                                     nullptr, s))
+                return rc;
+            e = launch_moe_swiglu(p.shared_g, p.shared_u, m * I, p.shared_act, s);
+            if (e != hipSuccess) return hip_fail(e, "MoE shared SwiGLU launch");
+            if (int rc = matmul_impl(&L->sdown, p.shared_act, m, p.shared_out, p.shared_ws, p.shared_ws_bytes,
+                                     IQ_PATH_AUTO, nullptr, nullptr, s))
+                return rc;
+        }
         e = launch_moe_shared_combine(x, L->selector, p.shared_out, residual, m, H, out, s);
         if (e != hipSuccess) return hip_fail(e, "MoE shared combine launch");
     }

@@ -38,11 +38,17 @@ struct QtArgs {
     int m;
     float* y;  // [m][ldy]
     int64_t ldy;
+    // a second matrix of the same shape over the same rows (blockIdx.z 1)
+    const uint8_t* w2 = nullptr;
+    float* y2 = nullptr;
 };
 
 // One wave per (row, 256 values): Q8_0 (bit-exact from_float).  The bytes
 // are stored + 128, the form bytes_to_f16 takes.
-__global__ __launch_bounds__(256) void k_qt_quant(const float* __restrict__ x, int64_t ldx, int64_t m, int64_t k,
+// SWIGLU: of SwiGLU(x, u) instead of x.
+template <bool SWIGLU>
+__global__ __launch_bounds__(256) void k_qt_quant(const float* __restrict__ x, const float* __restrict__ u, int64_t ldx,
+                                                  int64_t m, int64_t k,
                                                   int8_t* __restrict__ q, float* __restrict__ d) {
     const int lane = threadIdx.x & 63;
     const int64_t wid = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -50,7 +56,13 @@ __global__ __launch_bounds__(256) void k_qt_quant(const float* __restrict__ x, i
     if (wid >= m * ng) return;  // uniform per wave
     const int64_t row = wid / ng;
     const int g = (int)(wid - row * ng);
-    const Q80Lane r = quant_q80_core(q80_vals4_load(x + row * ldx, k, g));
+    f32x4 v = q80_vals4_load(x + row * ldx, k, g);
+    if constexpr (SWIGLU) {  // v is gate: (gate / (1 + exp(-gate))) * up, as the reference writes it
+        const f32x4 up = q80_vals4_load(u + row * ldx, k, g);
+#pragma unroll
+        for (int i = 0; i < 4; i++) v[i] = __fdiv_rn(v[i], 1.f + exp_f32(-v[i])) * up[i];
+    }
+    const Q80Lane r = quant_q80_core(v);
     const int64_t b = (int64_t)g * 8 + (lane >> 3);
     if (b >= k / 32) return;
     ((uint32_t*)(q + row * k + (int64_t)g * 256))[lane] = r.packed ^ 0x80808080u;
@@ -110,7 +122,7 @@ __global__ __launch_bounds__(512, 4) void k_qt_mm(QtArgs a) {
     const int tb = threadIdx.x, ta = NT - 1 - (int)threadIdx.x;
     const bool hasb = tb < kB, hasa = ta < kA;
     const int bc = tb & 3, ac = ta & 3, bcl = (tb >> 2) & (kQtCols - 1), arl = (ta >> 2) & (R - 1);
-    const uint8_t* bsrc = a.w + min(n0 + bcl, a.n - 1) * a.row_bytes + 34 * bc;
+    const uint8_t* bsrc = (blockIdx.z ? a.w2 : a.w) + min(n0 + bcl, a.n - 1) * a.row_bytes + 34 * bc;
     // quants from the aligned dword at or before them: an even block's start
     // two bytes into it (the ninth dword's upper half is the next block's),
     // an odd block's at it
@@ -222,11 +234,12 @@ __global__ __launch_bounds__(512, 4) void k_qt_mm(QtArgs a) {
         lds_barrier();
     }
     const int64_t n = n0 + cbase + jj;
+    float* y = blockIdx.z ? a.y2 : a.y;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const float v = ((acc[0][r] + acc[4][r]) + (acc[2][r] + acc[6][r])) + ((acc[1][r] + acc[5][r]) + (acc[3][r] + acc[7][r]));
         const int rr = rbase + 4 * q + r;
-        if (rr < rows && n < a.n) a.y[(int64_t)(row0 + rr) * a.ldy + n] = v;
+        if (rr < rows && n < a.n) y[(int64_t)(row0 + rr) * a.ldy + n] = v;
     }
 }
 
@@ -249,9 +262,9 @@ bool q8_tile_supported(const WeightView& w, int64_t m) {
     return !gemv_supported(w, m) || (double)(w.rows * w.row_bytes) * (double)m / 8 > 1e6 * (0.4 * (double)(w.cols / 32) - 4);
 }
 
-hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
-                          hipStream_t s) {
-    if (!q8_tile_supported(w, m)) return hipErrorNotSupported;
+namespace {
+
+QtArgs qt_args(const WeightView& w, int64_t m, void* ws) {
     QtArgs a;
     a.w = w.w;
     a.n = w.rows;
@@ -260,15 +273,55 @@ hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int6
     a.q = (const int8_t*)ws;
     a.d = (const float*)((uint8_t*)ws + align256((size_t)(m * w.cols)));
     a.m = (int)m;
+    a.ldy = w.rows;
+    return a;
+}
+
+template <bool SWIGLU>
+hipError_t qt_quant(const QtArgs& a, const float* x, const float* u, int64_t ldx, hipStream_t s) {
+    const int64_t k = (int64_t)a.nb * 32, waves = a.m * ((k + 255) / 256);
+    hipLaunchKernelGGL((k_qt_quant<SWIGLU>), dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, x, u, ldx, (int64_t)a.m, k,
+                       (int8_t*)a.q, (float*)a.d);
+    return hipGetLastError();
+}
+
+hipError_t qt_mm(const QtArgs& a, hipStream_t s) {
+    hipLaunchKernelGGL(k_qt_mm, dim3((unsigned)((a.n + kQtCols - 1) / kQtCols), (unsigned)((a.m + kQtRows - 1) / kQtRows),
+                                     a.w2 ? 2u : 1u), dim3(512), 0, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
+                          hipStream_t s) {
+    if (!q8_tile_supported(w, m)) return hipErrorNotSupported;
+    QtArgs a = qt_args(w, m, ws);
     a.y = y;
     a.ldy = ldy;
-    const int64_t qwaves = m * ((w.cols + 255) / 256);
-    hipLaunchKernelGGL(k_qt_quant, dim3((unsigned)((qwaves + 3) / 4)), dim3(256), 0, s, x, ldx, m, w.cols, (int8_t*)a.q,
-                       (float*)a.d);
-    if (hipError_t e = hipGetLastError()) return e;
-    hipLaunchKernelGGL(k_qt_mm, dim3((unsigned)((a.n + kQtCols - 1) / kQtCols), (unsigned)((m + kQtRows - 1) / kQtRows)),
-                       dim3(512), 0, s, a);
-    return hipGetLastError();
+    if (hipError_t e = qt_quant<false>(a, x, nullptr, ldx, s)) return e;
+    return qt_mm(a, s);
+}
+
+// Gate and up in one launch: apart, a [512 x 2048] matrix at 512 tokens is 128
+// workgroups, half the CUs, and takes as long as both together (19.6 us
+// each); x is quantised once, and SwiGLU runs inside the down product's
+// quantisation.  Four launches instead of seven: 1100 tokens 693 -> 616 us.
+hipError_t launch_q8_swiglu(const WeightView& gate, const WeightView& up, const WeightView& down, const float* x,
+                            int64_t m, float* g, float* u, float* out, void* ws, hipStream_t s) {
+    if (!q8_tile_supported(gate, m) || !q8_tile_supported(up, m) || !q8_tile_supported(down, m) ||
+        gate.rows != up.rows || gate.cols != up.cols || down.cols != gate.rows)
+        return hipErrorNotSupported;
+    QtArgs a = qt_args(gate, m, ws);
+    a.y = g;
+    a.w2 = up.w;
+    a.y2 = u;
+    if (hipError_t e = qt_quant<false>(a, x, nullptr, gate.cols, s)) return e;
+    if (hipError_t e = qt_mm(a, s)) return e;
+    QtArgs d = qt_args(down, m, ws);
+    d.y = out;
+    if (hipError_t e = qt_quant<true>(d, g, u, gate.rows, s)) return e;
+    return qt_mm(d, s);
 }
 
 }  // namespace iq

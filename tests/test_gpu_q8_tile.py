@@ -70,3 +70,30 @@ def test_nonfinite_scales_as_the_lane_kernel(gpu):
     assert np.array_equal(np.isnan(got), np.isnan(ref))
     ok = ~np.isnan(ref)
     assert np.array_equal(bits(got)[ok], bits(ref)[ok])
+
+
+@pytest.mark.parametrize("tokens", [9, 33, 70])
+@pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 512)])
+def test_q8_shared_expert_wide_equals_narrow(gpu, tokens, hidden, inter):
+    """A Q8_0 shared expert run apart: gate and up in one launch and SwiGLU inside down's quantisation give each token
+    what a call of up to 8 tokens (the lane kernel and the SwiGLU launch) gives it, bit for bit."""
+    import torch
+
+    from inferq_amd import moe as M, synth as S
+
+    rng = np.random.default_rng([tokens, hidden])
+    gate = down = S.Q4_K
+    layer = S.random_moe_layer(hidden, inter, 8, gate, down, rng)
+    for name, r, c in (("shared_gate", inter, hidden), ("shared_up", inter, hidden), ("shared_down", hidden, inter)):
+        layer[name] = S.random_matrix(S.Q8_0, r, c, rng)
+    t = {k: torch.from_numpy(v).to(gpu) for k, v in layer.items() if isinstance(v, np.ndarray)}
+    m = M.QuantizedMoeLayer(hidden, inter, 8, 2, gate, down, t["gate"], t["up"], t["down"], t["shared_gate"],
+                            t["shared_up"], t["shared_down"], t["selector"], shared_gate_dtype=S.Q8_0,
+                            shared_down_dtype=S.Q8_0)
+    x = torch.from_numpy(S.normal((tokens, hidden), rng)).to(gpu)
+    lg = torch.from_numpy(S.normal((tokens, 8), rng)).to(gpu)
+    wide, narrow = torch.empty_like(x), torch.empty_like(x)
+    m.forward_into(x, lg, wide)
+    for i in range(0, tokens, 8):
+        m.forward_into(x[i:i + 8].contiguous(), lg[i:i + 8].contiguous(), narrow[i:i + 8])
+    assert_bitexact(wide.cpu().numpy(), narrow.cpu().numpy(), f"{tokens} tokens")
