@@ -259,8 +259,7 @@ size_t matmul_ws_bytes(const iq_weight* w, int64_t m) {
     if (float_dtype(w->dtype)) return 0;  // the f32 product reads x as it is
     const size_t a = act_bytes(m, w->cols), p = prefill_workspace_size(view_of(w), m);
     const size_t d = dense_mfma_workspace_any(view_of(w), m);
-    const size_t ap = a > p ? a : p;
-    return ap > d ? ap : d;
+    return std::max({a, p, d, q8_few_workspace(view_of(w), m)});
 }
 
 // Greedy selection fused into the product (iq_matmul_argmax): 1 = one row
@@ -304,6 +303,8 @@ hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, 
         return path == IQ_PATH_AUTO && !isum ? launch_float_mm(v, x, w->cols, m, y, w->rows, s) : hipErrorNotSupported;
     if (path == IQ_PATH_AUTO) {
         if (!isum && dense_mfma_supported(v, m)) e = launch_dense_mfma(v, x, w->cols, m, y, w->rows, ws, s);
+        if (e == hipErrorNotSupported && !isum && q8_few_supported(v, m))
+            e = launch_q8_few(v, x, w->cols, m, y, w->rows, ws, s);
         if (e == hipErrorNotSupported && !isum && q8_tile_supported(v, m))
             e = launch_q8_tile(v, x, w->cols, m, y, w->rows, ws, s);
         if (e == hipErrorNotSupported && !isum && gemv_supported(v, m)) e = launch_gemv(v, x, w->cols, m, y, w->rows, s);

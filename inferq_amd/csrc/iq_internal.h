@@ -90,6 +90,14 @@ bool q8_tile_supported(const WeightView& w, int64_t m);
 hipError_t launch_q8_tile(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
                           hipStream_t s);
 
+// Q8_0 matrices at 3..8 input rows on f16 MFMA in the exact lane order
+// (iq_q8_tile.hip); quantises x itself into `ws` (at least q8_few_workspace
+// bytes, which do not fall as m grows).
+bool q8_few_supported(const WeightView& w, int64_t m);
+size_t q8_few_workspace(const WeightView& w, int64_t m);
+hipError_t launch_q8_few(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
+                         hipStream_t s);
+
 // out[m] = down . SwiGLU(gate . x, up . x) on Q8_0 matrices where
 // q8_tile_supported takes all three (else hipErrorNotSupported, nothing
 // launched); g and u [m][gate.rows], `ws` at least act_bytes of either width.

@@ -243,6 +243,136 @@ __global__ __launch_bounds__(512, 4) void k_qt_mm(QtArgs a) {
     }
 }
 
+// ---- 3..8 input rows --------------------------------------------------------
+//
+// v_mfma_f32_4x4x4_16b_f16 multiplies sixteen 4 x 4 by 4 x 4 pairs: here the
+// pairs are the eight reference lanes k times two groups of four input rows,
+// over four weight rows, so one instruction yields every lane's dot of a
+// block for 8 x 4 outputs and each lane of the wave holds four of them (lane
+// 8 k + 4 g + j: reference lane k, input rows 4 g .. 4 g + 3, weight row j).
+// A wave advances only four chains a block and decodes a weight once, where
+// the GEMV's waves keep eight rows' chains each.  What bounds it: one wave's
+// walk along its rows (about 200 cycles a block), and past 16000 rows the
+// VALU issue of the decode.  8 rows, GEMV before: [2048 x 4096] 17.2 -> 14.8
+// us, [8192 x 2048] 19.0 -> 13.2, [16000 x 4096] 52 -> 32.
+
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+constexpr int kQfSB = 32;                   // blocks per staged step of a weight row (1088 bytes)
+constexpr int kQfStride = 34 * kQfSB + 32;  // LDS row stride: four rows' dwords on distinct banks
+constexpr int kQfMaxNb = 128;               // blocks of the widest row (4096)
+
+struct QfArgs {
+    const uint8_t* w;  // [n][row_bytes], 16-byte aligned
+    int64_t n, row_bytes;
+    int nb;            // a multiple of kQfSB
+    const uint8_t* q;  // [nb / 2][64 lanes][16]: the lane's four values of two blocks as f16
+    const float* d;    // [nb][8] block scales
+    int m;
+    float* y;
+    int64_t ldy;
+};
+
+// One wave per (row of 8, 256 values); rows past m are zeros.
+__global__ __launch_bounds__(256) void k_qf_quant(const float* __restrict__ x, int64_t ldx, int m, int64_t k,
+                                                  uint8_t* __restrict__ q, float* __restrict__ d) {
+    const int lane = threadIdx.x & 63;
+    const int wid = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), ng = (int)(k / 256);
+    if (wid >= 8 * ng) return;  // uniform per wave
+    const int row = wid / ng, g = wid - row * ng;
+    Q80Lane r = {0u, 0};
+    if (row < m) r = quant_q80_core(q80_vals4_load(x + row * ldx, k, g));
+    const int b = 8 * g + (lane >> 3), kk = lane & 7;
+    *(u32x2*)(q + ((int64_t)(b >> 1) * 64 + 8 * kk + row) * 16 + 8 * (b & 1)) = bytes_to_f16(r.packed ^ 0x80808080u);
+    if (kk == 0) d[b * 8 + row] = f16_to_f32(r.dh);
+}
+
+// Grid n / 8: a workgroup of two waves, four weight rows each.
+__global__ __launch_bounds__(128) void k_qf_mm(QfArgs a) {
+    __shared__ __align__(16) uint8_t st[2][2][4 * kQfStride];  // [wave][step]
+    __shared__ __align__(16) float s_d[kQfMaxNb * 8];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int j = lane & 3, g = (lane >> 2) & 1, k = lane >> 3;
+    const int64_t n0 = ((int64_t)blockIdx.x * 2 + wave) * 4;
+    // a step's 4 rows x 68 granules of 16 bytes, five loads a lane
+    constexpr int kG = 34 * kQfSB / 16, kL = (4 * kG + 63) / 64;
+    const uint8_t* src[kL];
+    int dst[kL];
+#pragma unroll
+    for (int i = 0; i < kL; i++) {
+        const int t = min(lane + 64 * i, 4 * kG - 1), r = t / kG, part = t - r * kG;
+        src[i] = a.w + min(n0 + r, a.n - 1) * a.row_bytes + 16 * part;
+        dst[i] = r * kQfStride + 16 * part;
+    }
+    u32x4 sb[kL];
+    auto issue = [&](int s) {
+#pragma unroll
+        for (int i = 0; i < kL; i++) sb[i] = *(const u32x4*)(src[i] + (int64_t)s * (34 * kQfSB));
+    };
+    auto park = [&](int p) {
+#pragma unroll
+        for (int i = 0; i < kL; i++) *(u32x4a16*)(st[wave][p] + dst[i]) = u32x4a16{sb[i].x, sb[i].y, sb[i].z, sb[i].w};
+    };
+    const int ns = a.nb / kQfSB;
+    issue(0);
+    u32x4a16 av[2][4];  // the activations of four blocks pairs, two sets
+    const uint8_t* aq = a.q + 16 * lane;
+    auto fetch = [&](int pair, u32x4a16 (&o)[4]) {  // pairs past the end are never used: clamp
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i] = *(const u32x4a16*)(aq + (int64_t)min(pair + i, a.nb / 2 - 1) * 1024);
+    };
+    fetch(0, av[0]);
+    for (int i = threadIdx.x; i < a.nb * 2; i += 128) ((f32x4*)s_d)[i] = ((const f32x4*)a.d)[i];
+    park(0);
+    __syncthreads();
+    float acc[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < ns; s++) {
+        if (s + 1 < ns) issue(s + 1);
+        const uint8_t* row = st[wave][s & 1] + j * kQfStride;
+        const float* dp = s_d + (s * kQfSB) * 8 + 4 * g;
+        // a real loop over halves of a step: unrolled whole, the operands of its 32 blocks were live at once
+        // (362 registers a lane against 116, half the waves: [16000 x 2048] at 8 rows 28.5 -> 19.7 us)
+#pragma unroll 1
+        for (int h = 0; h < kQfSB; h += 16, row += 16 * 34, dp += 16 * 8) {
+#pragma unroll
+            for (int c = 0; c < 16; c++) {
+                if (c % 8 == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch((s * kQfSB + h + c) / 2 + 4, av[(c / 8 + 1) & 1]);
+                }
+                const uint32_t lo = *(const uint32_t*)(row + ((34 * c) & ~3) + 4 * k);
+                const uint32_t hi = *(const uint32_t*)(row + ((34 * c) & ~3) + 4 * k + 4);
+                // quants at 2 (mod 4) in an even block, aligned (the second dword) in an odd one
+                const uint32_t v = (c & 1) ? hi : __builtin_amdgcn_alignbyte(hi, lo, 2);
+                const float xd = f16_to_f32(*(const uint16_t*)(row + 34 * c));
+                const u32x4a16 aw = av[(c / 8) & 1][(c & 7) >> 1];
+                const v4h af = __builtin_bit_cast(v4h, (c & 1) ? u32x2{aw.z, aw.w} : u32x2{aw.x, aw.y});
+                const v4h bf = __builtin_bit_cast(v4h, bytes_to_f16(v ^ 0x80808080u));
+                const v4f z = {};
+                const v4f dot = __builtin_amdgcn_mfma_f32_4x4x4f16(af, bf, z, 0, 0, 0);
+                const f32x4 yd = *(const f32x4*)(dp + 8 * c);
+#pragma unroll
+                for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(xd * yd[r], dot[r], acc[r]);
+            }
+        }
+        if (s + 1 < ns) park((s + 1) & 1);
+        // the step's region is this wave's own
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    // hsum_f32_8 over lanes k (bits 3..5 of the lane)
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        float v = acc[r];
+        v = v + __shfl_xor(v, 32);
+        v = v + __shfl_xor(v, 16);
+        v = v + __shfl_xor(v, 8);
+        const int rr = 4 * g + r;
+        if (k == 0 && rr < a.m && n0 + j < a.n) a.y[(int64_t)rr * a.ldy + n0 + j] = v;
+    }
+}
+
 constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 }  // namespace
@@ -322,6 +452,56 @@ hipError_t launch_q8_swiglu(const WeightView& gate, const WeightView& up, const 
     d.y = out;
     if (hipError_t e = qt_quant<true>(d, g, u, gate.rows, s)) return e;
     return qt_mm(d, s);
+}
+
+namespace {
+
+// What k_qf_* can take at any number of rows up to 8.
+bool qf_shape(const WeightView& w) {
+    return w.dtype == kQ8_0 && w.rows >= 1 && w.rows <= (int64_t)1 << 31 && w.cols >= 1 && w.cols % (32 * kQfSB) == 0 &&
+           w.cols / 32 <= kQfMaxNb && ((uintptr_t)w.w & 15) == 0;
+}
+
+}  // namespace
+
+// The tile's time hardly depends on the rows; the GEMV's grows with them and
+// with the matrix, so the line is a least amount of work that falls with the
+// row's length (a chain's walk: 0.09 us a block).  Measured, tile / GEMV in
+// us: [2048 x 4096] at 6 / 7 rows 14.9 / 14.5 and 14.8 / 17.2, [4096 x 4096]
+// at 3 / 4 rows 17.0 / 15.0 and 17.1 / 18.1, [4096 x 2048] at 4 / 5 rows 11.3
+// / 11.0 and 11.4 / 14.5, [2048 x 1024] at 8 rows 7.6 / 7.5, [8192 x 1024] at
+// 5 rows 9.4 / 11.5.  Past 16384 rows the GEMV's waves fill the chip and it
+// reads the matrix at a better rate: [16000 x 2048] at 3 rows 19.4 / 24.9,
+// [24576 x 2048] at 4 rows 24.3 / 22.1, [32000 x 2048] at 4 / 6 rows 30.9 /
+// 29.1 and 29.1 / 34.0, [248320 x 2048] at 6 / 8 rows 177 / 163 and 177 / 199.
+// Rows of 6144: 20.4 / 17.9 at 8 rows, so not taken.
+bool q8_few_supported(const WeightView& w, int64_t m) {
+    if (m < 3 || m > 8 || !qf_shape(w)) return false;
+    return m >= (w.rows <= 16384 ? 3 : w.rows <= 65536 ? 6 : 8) && w.rows * m * (w.cols / 32 + 64) >= 2500000;
+}
+
+size_t q8_few_workspace(const WeightView& w, int64_t m) {
+    return m >= 3 && qf_shape(w) ? (size_t)w.cols * 17 : 0;
+}
+
+hipError_t launch_q8_few(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, void* ws,
+                         hipStream_t s) {
+    if (!q8_few_supported(w, m)) return hipErrorNotSupported;
+    QfArgs a;
+    a.w = w.w;
+    a.n = w.rows;
+    a.row_bytes = w.row_bytes;
+    a.nb = (int)(w.cols / 32);
+    a.q = (const uint8_t*)ws;
+    a.d = (const float*)((uint8_t*)ws + w.cols * 16);
+    a.m = (int)m;
+    a.y = y;
+    a.ldy = ldy;
+    hipLaunchKernelGGL(k_qf_quant, dim3((unsigned)(w.cols / 128)), dim3(256), 0, s, x, ldx, (int)m, w.cols, (uint8_t*)a.q,
+                       (float*)a.d);
+    if (hipError_t e = hipGetLastError()) return e;
+    hipLaunchKernelGGL(k_qf_mm, dim3((unsigned)((a.n + 7) / 8)), dim3(128), 0, s, a);
+    return hipGetLastError();
 }
 
 }  // namespace iq

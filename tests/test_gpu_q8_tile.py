@@ -33,6 +33,28 @@ def test_tile_edges_bitwise(gpu, oracle, rows, cols, m):
     assert_bitexact(got, oracle.matmul(S.Q8_0, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
 
 
+# 3..8 rows: either side of the rule's lines (the GEMV takes the other), ragged row counts, one to four steps of 1024
+@pytest.mark.parametrize("rows,cols,m", [(8681, 1024, 3), (8680, 1024, 3), (6511, 1024, 4), (3256, 1024, 8),
+                                         (2443, 2048, 8), (3907, 2048, 5), (2051, 3072, 8), (1862, 4096, 7),
+                                         (1629, 4096, 8), (1628, 4096, 8), (16384, 1024, 3), (16385, 1024, 3),
+                                         (16385, 1024, 6), (65537, 1024, 8), (2000, 5120, 8)])
+def test_few_rows_bitwise(gpu, oracle, rows, cols, m):
+    import torch
+
+    from inferq_amd import synth as S
+
+    rng = np.random.default_rng([rows, cols, m])
+    w, mat = _mat(rows, cols, rng)
+    x = S.normal((m, cols), rng)
+    x[0] = 0.0
+    x[m - 1] *= np.float32(1e-20)
+    x[1, :32] = np.where(np.arange(32) % 2, np.float32(-3), np.float32(3))
+    out = torch.full((m + 1, rows), 7.0, device=gpu)
+    mat.forward_into(torch.from_numpy(x).to(gpu), out[:m])
+    assert torch.all(out[m] == 7.0)
+    assert_bitexact(out[:m].cpu().numpy(), oracle.matmul(S.Q8_0, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
+
+
 @pytest.mark.parametrize("fill", [0x80, 0x7F, 0xFF, 0x00])
 def test_extreme_values_bitwise(gpu, oracle, fill):
     """Every weight byte -128, 127, -1 or 0 against rows that quantise to +-127."""
@@ -51,13 +73,13 @@ def test_extreme_values_bitwise(gpu, oracle, fill):
     assert_bitexact(got, oracle.matmul(S.Q8_0, w.reshape(-1), rows, cols, x), f"bytes {fill:#x}")
 
 
-def test_nonfinite_scales_as_the_lane_kernel(gpu):
+@pytest.mark.parametrize("rows,cols,m", [(66, 384, 35), (3260, 1024, 8)])
+def test_nonfinite_scales_as_the_lane_kernel(gpu, rows, cols, m):
     """Infinities and NaN in rows and in weight scales: NaN where the lane kernel has NaN, its bits elsewhere."""
     import torch
 
     from inferq_amd import _lib, qgemm as Q, synth as S
 
-    rows, cols, m = 66, 384, 35
     rng = np.random.default_rng(5)
     w = S.random_matrix(S.Q8_0, rows, cols, rng).reshape(rows, -1, 34)
     w[3, 2, 0:2] = np.array([0x7C00], np.uint16).view(np.uint8)  # inf
