@@ -78,7 +78,7 @@ enum iq_path {
     IQ_PATH_AUTO = 0,
     IQ_PATH_LANES = 1,        /* generic lane kernel (any dtype, any m) */
     IQ_PATH_GEMV = 2,         /* LDS-staged GEMV (1..63 rows, K-quant and Q8_0) */
-    IQ_PATH_LANE_MFMA = 3,    /* exact lane order on int8 MFMA (Q4_K / Q6_K) */
+    IQ_PATH_LANE_MFMA = 3,    /* exact lane order on MFMA (Q4_K / Q5_K / Q6_K) */
     IQ_PATH_PREFILL_TILES = 4 /* tile-order int8 MFMA (Q4_K, m >= 64): NOT bitwise */
 };
 

@@ -102,17 +102,16 @@ __global__ __launch_bounds__(256) void k_dh_mm(DmArgs a) {
     }
 }
 
-// The same on int8 MFMA, with k_dm_quant's activations.
-template <int FMT, int RT>
+// Q6_K, 16 input rows per workgroup, on int8 MFMA with k_dm_quant's activations.
 __global__ __launch_bounds__(256) void k_dm_mm(DmArgs a) {
-    using L = MlStage<FMT, RT>;
+    using L = MlStage<kQ6_K, 1>;
     __shared__ __align__(16) uint8_t st[2][L::END];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, jj = lane & 15;
     const int64_t n0 = (int64_t)blockIdx.x * kMlCols;
-    const int row0 = (int)blockIdx.y * 16 * RT;
-    const int rows = min(16 * RT, a.m - row0);
+    const int row0 = (int)blockIdx.y * 16;
+    const int rows = min(16, a.m - row0);
     MlOperands op;
     op.aq = a.q;
     op.ldq = (int64_t)a.nb * 256;
@@ -126,12 +125,12 @@ __global__ __launch_bounds__(256) void k_dm_mm(DmArgs a) {
     const int64_t last = a.n - 1 - n0;
     auto brow = [&](int t) -> int64_t { return t < last ? (int64_t)t : last; };
     auto arow = [&](int rr) -> int64_t { return row0 + min(rr, rows - 1); };
-    float v[4 * RT];
-    ml_product<FMT, RT>(op, arow, brow, st, v);
+    float v[4];
+    ml_product(op, arow, brow, st, v);
     const int64_t n = n0 + 16 * wave + jj;
 #pragma unroll
-    for (int r = 0; r < 4 * RT; r++) {
-        const int rr = 16 * (r >> 2) + 4 * q + (r & 3);
+    for (int r = 0; r < 4; r++) {
+        const int rr = 4 * q + r;
         if (rr < rows && n < a.n) a.y[(int64_t)(row0 + rr) * a.ldy + n] = v[r];
     }
 }
@@ -302,10 +301,9 @@ hipError_t launch_h(const DmArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int FMT, int RT>
-hipError_t launch_t(const DmArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)((a.n + kMlCols - 1) / kMlCols), (unsigned)((a.m + 16 * RT - 1) / (16 * RT)));
-    hipLaunchKernelGGL((k_dm_mm<FMT, RT>), grid, dim3(256), 0, s, a);
+hipError_t launch_q6(const DmArgs& a, hipStream_t s) {
+    const dim3 grid((unsigned)((a.n + kMlCols - 1) / kMlCols), (unsigned)((a.m + 15) / 16));
+    hipLaunchKernelGGL(k_dm_mm, grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -401,7 +399,7 @@ hipError_t launch_dense_argmax(const WeightView& w, const float* x, int64_t m, f
 
 template <int FMT>
 static hipError_t dense_tiles(const DmArgs& a, bool rt1, hipStream_t s) {
-    if constexpr (FMT == kQ6_K) return rt1 ? launch_t<FMT, 1>(a, s) : launch_h<FMT, 2>(a, s);
+    if constexpr (FMT == kQ6_K) return rt1 ? launch_q6(a, s) : launch_h<FMT, 2>(a, s);
     else return rt1 ? launch_h<FMT, 1>(a, s) : launch_h<FMT, 2>(a, s);
 }
 

@@ -71,7 +71,7 @@ size_t prefill_workspace_size(const WeightView& w, int64_t m);
 hipError_t launch_prefill(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
                           void* ws, int32_t* dbg_isum, int32_t* dbg_msum, hipStream_t s);
 
-// The exact lane-order int8-MFMA kernel for Q4_K / Q6_K matrices
+// The exact lane-order MFMA kernels for Q4_K / Q5_K / Q6_K matrices
 // (iq_dense_mfma.hip): bitwise the one-row results.  dense_mfma_supported
 // says where the dispatch uses it (large matrices at 2..63 input rows, every
 // readable matrix from kPrefillMinRows rows); launch_dense_mfma_any runs it

@@ -1,7 +1,7 @@
 // iq_mfma_lanes.h -- the reference's exact per-lane products on int8 MFMA
 // (Q4_K or Q6_K weights), shared by the grouped MoE kernels and the dense
-// multi-row kernels, in three forms:
-//   ml_product     up to 16 RT activation rows x 64 weight rows;
+// multi-row kernels, in three forms (wider tiles: iq_mfma_half.h):
+//   ml_product     up to 16 activation rows x 64 weight rows, Q6_K;
 //   ml_product_pk  up to 8 activation rows x 64 weight rows, two reference
 //                  lanes per v_mfma_i32_16x16x64_i8;
 //   ml_product_sk  up to 8 activation rows x 16 weight rows, the blocks
@@ -18,10 +18,7 @@
 // folded in.  Scaled weights exceed int8, so each is split into two int8
 // streams whose integer sums recombine exactly: Q4_K sc*q = 8 (sc >> 3) q +
 // (sc & 7) q; Q6_K sc*(q - 32) = 256 hi + lo with hi in -16..16 and lo in
-// -128..127; Q5_K (q = nibble + 16 bit) into three, 8 (sc >> 3) nibble +
-// (sc & 7) nibble + 16 sc bit.  Q5_K's mins join one f32 scalar per row
-// and block, summs = summs + dmin * (m . s) (ggml's vec_dot_q5_K_q8_K), the
-// integer m . s from one f16 MFMA (exact: integers below 2^24).  The Q4_K mins msum_k = m_2k s_2k + m_2k+1 s_2k+1 (s = 32-value
+// -128..127.  The Q4_K mins msum_k = m_2k s_2k + m_2k+1 s_2k+1 (s = 32-value
 // activation sums) come from an f16 MFMA over the 16-value sums (integers
 // below 2^24: exact).  A lane keeps the f32 chains of all eight reference
 // lanes for its outputs and joins them at the end in the hsum trees' order,
@@ -51,7 +48,7 @@ struct MlFmt<kQ4_K> {
     static constexpr int NL = 9;    // staging loads per row-block (16 bytes each)
     static constexpr bool kMins = true;
 };
-// Q5_K (ml_product only): the Q4_K header, qh at 16..47, qs at 48..175;
+// Q5_K (iq_mfma_half.h): the Q4_K header, qh at 16..47, qs at 48..175;
 // 176-byte columns (11 groups of 16 bytes, coprime with the 16 bank groups)
 template <>
 struct MlFmt<kQ5_K> {
@@ -185,18 +182,20 @@ struct MlOperands {
 };
 
 // The tile's products on a 256-thread workgroup: lane (q = l / 16, j = l % 16)
-// of wave w ends with v[r] = output (row 16 (r / 4) + 4 q + r % 4, weight
-// row 16 w + j), r < 4 RT.  `st` is the caller's LDS (2 stages).
+// of wave w ends with v[r] = output (row 4 q + r, weight row 16 w + j).  `st`
+// is the caller's LDS (2 stages).  Q6_K only: the other formats, and Q6_K at
+// 32 rows, run on f16 MFMA, which at 16 rows loses to this on Q6_K (its decode
+// there is the larger; the [248320 x 2048] head at 16 rows 123 us for 115).
 //
 // Fragments of v_mfma_i32_16x16x32_i8 for lane l (q = l / 16, j = l % 16):
 // A row j, K 8q..8q+7; B column j, the same K; the result holds rows
 // 4q..4q+3 of column j.  For lane k of the reference, K 8q..8q+7 are the
 // dwords (c, k) with c = 2q, 2q+1.
-template <int FMT, int RT, class ARow, class BRow>
-__device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow brow, uint8_t (*st)[MlStage<FMT, RT>::END],
-                                           float (&v)[4 * RT]) {
-    using F = MlFmt<FMT>;
-    using L = MlStage<FMT, RT>;
+template <class ARow, class BRow>
+__device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow brow,
+                                           uint8_t (*st)[MlStage<kQ6_K, 1>::END], float (&v)[4]) {
+    using F = MlFmt<kQ6_K>;
+    using L = MlStage<kQ6_K, 1>;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, jj = lane & 15;
@@ -204,21 +203,14 @@ __device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow
 
     // ---- staging: every thread owns fixed slots, the same for every block.
     // Sources are a wave-uniform base plus a 32-bit offset.
-    constexpr int kA = L::R * 16;              // 16-byte A chunks
-    constexpr int kB = kMlCols * F::NL;        // 16-byte B chunks
-    constexpr int kAPer = (kA + 255) / 256;    // 1 or 2
-    constexpr int kBPer = (kB + 255) / 256;    // Q4_K 3, Q6_K 4
-    uint32_t a_src[kAPer];
-    int a_off[kAPer];
-#pragma unroll
-    for (int i = 0; i < kAPer; i++) {
-        const int t = min((int)threadIdx.x + 256 * i, kA - 1);
-        const int rr = t >> 4, part = t & 15;
-        a_src[i] = (uint32_t)(arow(rr) * op.ldq + 16 * part);
-        a_off[i] = (int)threadIdx.x + 256 * i < kA ? L::A + rr * kMlAS + 16 * part : -1;
-    }
+    static_assert(L::R * 16 == 256, "one 16-byte A chunk per thread");
+    constexpr int kB = kMlCols * F::NL;      // 16-byte B chunks
+    constexpr int kBPer = (kB + 255) / 256;  // 4
+    const int a_rr = threadIdx.x >> 4, a_part = threadIdx.x & 15;
+    const uint32_t a_src = (uint32_t)(arow(a_rr) * op.ldq + 16 * a_part);
+    const int a_off = L::A + a_rr * kMlAS + 16 * a_part;
     // B chunk t: column t / NL, part t % NL; columns past bsplit come from
-    // the second matrix.  Q6_K: the block's dword window (it starts 0 or 2
+    // the second matrix.  The block's dword window (it starts 0 or 2
     // bytes before the block) as 13 chunks plus one ending at its last byte.
     uint32_t b_src[kBPer];
     int b_off[kBPer];
@@ -227,216 +219,93 @@ __device__ __forceinline__ void ml_product(const MlOperands& op, ARow arow, BRow
     for (int i = 0; i < kBPer; i++) {
         const int t = min((int)threadIdx.x + 256 * i, kB - 1);
         const int c2 = t / F::NL, part = t - c2 * F::NL;
-        const int po = FMT == kQ6_K && part == F::NL - 1 ? 196 : 16 * part;
+        const int po = part == F::NL - 1 ? 196 : 16 * part;
         b_hi[i] = c2 >= op.bsplit;
         b_last[i] = part == F::NL - 1;
         b_src[i] = (uint32_t)(brow(c2) * op.brow_bytes + po);
         b_off[i] = (int)threadIdx.x + 256 * i < kB ? L::B + c2 * F::BS + po : -1;
     }
-    // D (row scales) on threads 0 .. R-1, H (16-value sums, Q4_K) on 64 .. 64 + 2R - 1
-    static_assert((L::R & (L::R - 1)) == 0, "tile rows");
-    const int tD = threadIdx.x, tH = threadIdx.x - 64;
+    const int tD = threadIdx.x;  // D (row scales) on threads 0 .. 15
     const int64_t d_row = arow(tD & (L::R - 1));
-    const int64_t h_row = arow((tH >> 1) & (L::R - 1));  // in range for idle threads too
 
-    v4i_ml sa[kAPer];
+    v4i_ml sa;
     u32x4 sb[kBPer];
     float sd = 0.f;
-    v4i_ml sh16 = {};
     auto issue = [&](int b) {
-        const int8_t* abase = op.aq + (int64_t)b * 256;
-#pragma unroll
-        for (int i = 0; i < kAPer; i++) sa[i] = *(const v4i_ml*)(abase + a_src[i]);
-        const int64_t boff = FMT == kQ6_K ? ((int64_t)b * F::BB) & ~(int64_t)3 : (int64_t)b * F::BB;
+        sa = *(const v4i_ml*)(op.aq + (int64_t)b * 256 + a_src);
+        const int64_t boff = ((int64_t)b * F::BB) & ~(int64_t)3;
 #pragma unroll
         for (int i = 0; i < kBPer; i++) sb[i] = *(const u32x4*)((b_hi[i] ? op.b1 : op.b0) + boff + b_src[i]);
         if (tD < L::R) sd = op.ad[d_row * op.ldd + b];
-        if constexpr (F::kMins)
-            if (tH >= 0 && tH < 2 * L::R) sh16 = *(const v4i_ml*)(op.hs + (h_row * nb + b) * 16 + 8 * (tH & 1));
     };
     auto park = [&](uint8_t* s) {
-#pragma unroll
-        for (int i = 0; i < kAPer; i++)
-            if (a_off[i] >= 0) *(v4i_ml*)(s + a_off[i]) = sa[i];
+        *(v4i_ml*)(s + a_off) = sa;
 #pragma unroll
         for (int i = 0; i < kBPer; i++)
-            if (b_off[i] >= 0) ml_park_b<FMT>(s + b_off[i], sb[i], b_last[i]);
+            if (b_off[i] >= 0) ml_park_b<kQ6_K>(s + b_off[i], sb[i], b_last[i]);
         if (tD < L::R) *(float*)(s + L::D + 4 * tD) = sd;
-        if constexpr (F::kMins)
-            if (tH >= 0 && tH < 2 * L::R) *(v4i_ml*)(s + L::H + 32 * (tH >> 1) + 16 * (tH & 1)) = sh16;
     };
 
     const int col = 16 * wave + jj;  // this lane's staged weight row
-    // output r of the lane: tile r / 4, row 16 (r / 4) + 4 q + r % 4;
-    // acc[k]: the f32 chain of reference lane k, accm[k] of mins lane k
-    float acc[8][4 * RT], accm[4][4 * RT];
+    float acc[8][4];  // acc[k]: the f32 chain of reference lane k
 #pragma unroll
     for (int k = 0; k < 8; k++)
 #pragma unroll
-        for (int r = 0; r < 4 * RT; r++) acc[k][r] = 0.f;
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-#pragma unroll
-        for (int r = 0; r < 4 * RT; r++) accm[k][r] = 0.f;
+        for (int r = 0; r < 4; r++) acc[k][r] = 0.f;
     issue(0);
     park(st[0]);
     lds_barrier();
     for (int b = 0; b < nb; b++) {
         const uint8_t* S = st[b & 1];
         if (b + 1 < nb) issue(b + 1);
-        const int sh = FMT == kQ6_K ? (int)(((int64_t)b * F::BB) & 3) : 0;
+        const int sh = (int)(((int64_t)b * F::BB) & 3);
         const uint8_t* bcol = S + L::B + col * F::BS;
-        float dd[4 * RT], dm[4 * RT];
-        float xd, xdm = 0.f;
-        uint32_t s6a = 0, s6b = 0;  // Q4_K: six-bit scales of sub-blocks 2q, 2q+1
-        uint32_t q6s = 0;           // Q6_K: scale bytes 4q..4q+3
-        Q4Scales sc{};
-        // Q4_K: the lane's qs bytes 32q .. 32q + 31 (dword k for reference
-        // lane k), read as two 16-byte LDS accesses per block: the
-        // columns' 144-byte stride puts 16 lanes' 16-byte groups on 16
-        // distinct bank groups, where eight 4-byte reads per block would
-        // put four lanes on each bank
-        u32x4a16 qs4[2] = {};
-        u32x4a16 qh4[2] = {};  // Q5_K: qh bytes 0..31 (dword k: the fifth bits of lane k)
-        // Q6_K: the lane's ql and qh windows for reference lanes k = 0..7
-        uint32_t l0s[8] = {}, l1s[8] = {}, qhs[8] = {};
-        if constexpr (FMT == kQ4_K || FMT == kQ5_K) {
-            constexpr int QO = FMT == kQ5_K ? 48 : 16;  // offset of qs
-            const u32x4a16 hdr = *(const u32x4a16*)bcol;
-            xd = f16_to_f32(hdr.x);
-            xdm = f16_to_f32(hdr.x >> 16);
-            sc = q4_scales(hdr.y, hdr.z, hdr.w);
-            const uint32_t sw = q < 2 ? sc.sc_lo : sc.sc_hi;
-            s6a = byte_of(sw, 2 * (q & 1));
-            s6b = byte_of(sw, 2 * (q & 1) + 1);
-            qs4[0] = *(const u32x4a16*)(bcol + QO + 32 * q);
-            qs4[1] = *(const u32x4a16*)(bcol + QO + 16 + 32 * q);
-            if constexpr (FMT == kQ5_K) {
-                qh4[0] = *(const u32x4a16*)(bcol + 16);
-                qh4[1] = *(const u32x4a16*)(bcol + 32);
-            }
-        } else {
-            xd = f16_to_f32(ml_lds_win(bcol, sh, 208) & 0xffffu);
-            q6s = ml_lds_win(bcol, sh, 192 + 4 * q);
-            ml_lds_span<8>(bcol, sh, 64 * (q >> 1), l0s);
-            ml_lds_span<8>(bcol, sh, 64 * (q >> 1) + 32, l1s);
-            ml_lds_span<8>(bcol, sh, 128 + 32 * (q >> 1), qhs);
-        }
+        const float xd = f16_to_f32(ml_lds_win(bcol, sh, 208) & 0xffffu);
+        const uint32_t q6s = ml_lds_win(bcol, sh, 192 + 4 * q);  // scale bytes 4q..4q+3
+        // the lane's ql and qh windows for reference lanes k = 0..7
+        uint32_t l0s[8], l1s[8], qhs[8];
+        ml_lds_span<8>(bcol, sh, 64 * (q >> 1), l0s);
+        ml_lds_span<8>(bcol, sh, 64 * (q >> 1) + 32, l1s);
+        ml_lds_span<8>(bcol, sh, 128 + 32 * (q >> 1), qhs);
+        float dd[4];
 #pragma unroll
-        for (int r = 0; r < 4 * RT; r++) {
-            const float yd = *(const float*)(S + L::D + 4 * (16 * (r >> 2) + 4 * q + (r & 3)));
-            dd[r] = yd * xd;
-            if constexpr (F::kMins) dm[r] = -yd * xdm;
-        }
+        for (int r = 0; r < 4; r++) dd[r] = *(const float*)(S + L::D + 4 * (4 * q + r)) * xd;
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-            uint32_t w1[2], w2[2], w3[2] = {0u, 0u};
-            int mul;  // isum = mul * (stream 1) + (stream 2) (+ 16 * (stream 3), Q5_K)
-            if constexpr (FMT == kQ4_K || FMT == kQ5_K) {
-                const uint32_t qd = qs4[k >> 2][k & 3];
-                const uint32_t lo = qd & 0x0f0f0f0fu, hi = (qd >> 4) & 0x0f0f0f0fu;
-                w1[0] = bytes_mul_small(lo, s6a >> 3);
-                w1[1] = bytes_mul_small(hi, s6b >> 3);
-                w2[0] = bytes_mul_small(lo, s6a & 7u);
-                w2[1] = bytes_mul_small(hi, s6b & 7u);
-                if constexpr (FMT == kQ5_K) {
-                    // fifth bits of chunks 2q, 2q + 1 (bits 2q, 2q + 1 of
-                    // qh bytes 4k .. 4k + 3), each byte 0 or the scale
-                    const uint32_t qhd = qh4[k >> 2][k & 3];
-                    w3[0] = bytes_mul_small((qhd >> (2 * q)) & 0x01010101u, s6a);
-                    w3[1] = bytes_mul_small((qhd >> (2 * q + 1)) & 0x01010101u, s6b);
-                }
-                mul = 8;
-            } else {
-                const int hk = k >= 4;
-                const uint32_t l0 = l0s[k], l1 = l1s[k], qh = qhs[k];
+            uint32_t w1[2], w2[2];  // isum = 256 * (stream 1) + (stream 2)
+            const int hk = k >= 4;
+            const uint32_t l0 = l0s[k], l1 = l1s[k], qh = qhs[k];
 #pragma unroll
-                for (int cc = 0; cc < 2; cc++) {
-                    const uint32_t l = cc ? l1 : l0;
-                    const uint32_t lo4 = (q & 1) ? ((l >> 4) & 0x0f0f0f0fu) : (l & 0x0f0f0f0fu);
-                    const uint32_t u = lo4 | (((qh >> (2 * (2 * (q & 1) + cc))) & 0x03030303u) << 4);
-                    const int scv = (int)(int8_t)(uint8_t)(q6s >> (8 * (2 * cc + hk)));
-                    ml_q6_scaled_split(u, scv, w2[cc], w1[cc]);
-                }
-                mul = 256;
+            for (int cc = 0; cc < 2; cc++) {
+                const uint32_t l = cc ? l1 : l0;
+                const uint32_t lo4 = (q & 1) ? ((l >> 4) & 0x0f0f0f0fu) : (l & 0x0f0f0f0fu);
+                const uint32_t u = lo4 | (((qh >> (2 * (2 * (q & 1) + cc))) & 0x03030303u) << 4);
+                const int scv = (int)(int8_t)(uint8_t)(q6s >> (8 * (2 * cc + hk)));
+                ml_q6_scaled_split(u, scv, w2[cc], w1[cc]);
             }
             const long b1 = (long)(((uint64_t)w1[1] << 32) | w1[0]);
             const long b2 = (long)(((uint64_t)w2[1] << 32) | w2[0]);
-            const long b3 = (long)(((uint64_t)w3[1] << 32) | w3[0]);
+            const long a = *(const long*)(S + L::A + jj * kMlAS + 32 * k + 8 * q);
+            const v4i_ml z = {};
+            const v4i_ml i1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b1, z, 0, 0, 0);
+            const v4i_ml i2 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b2, z, 0, 0, 0);
 #pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const long a = *(const long*)(S + L::A + (16 * t + jj) * kMlAS + 32 * k + 8 * q);
-                const v4i_ml z = {};
-                const v4i_ml i1 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b1, z, 0, 0, 0);
-                const v4i_ml i2 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b2, z, 0, 0, 0);
-                v4i_ml i3 = z;
-                if constexpr (FMT == kQ5_K) i3 = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b3, z, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    int32_t isum = i1[r] * mul + i2[r];
-                    if constexpr (FMT == kQ5_K) isum += 16 * i3[r];
-                    acc[k][4 * t + r] = __builtin_fmaf(dd[4 * t + r], (float)isum, acc[k][4 * t + r]);
-                }
-            }
+            for (int r = 0; r < 4; r++) acc[k][r] = __builtin_fmaf(dd[r], (float)(i1[r] * 256 + i2[r]), acc[k][r]);
             // one lane's products at a time: the chains are advanced here
             // (not sunk to the end of the block), which bounds the live
             // MFMA results
 #pragma unroll
-            for (int r = 0; r < 4 * RT; r++) asm volatile("" : "+v"(acc[k][r]));
+            for (int r = 0; r < 4; r++) asm volatile("" : "+v"(acc[k][r]));
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if constexpr (FMT == kQ5_K) {
-            // m . s over the whole block in one f16 MFMA (lane group q
-            // supplies mins 2q, 2q + 1 against 16-value sums 4q .. 4q + 3),
-            // then summs = summs + dmin * (m . s) per row, held in accm[0]
-            const uint32_t mwd = q < 2 ? sc.mn_lo : sc.mn_hi;
-            const _Float16 mA = (_Float16)(float)byte_of(mwd, 2 * (q & 1));
-            const _Float16 mB = (_Float16)(float)byte_of(mwd, 2 * (q & 1) + 1);
-            const v4h_ml bm = {mA, mA, mB, mB};
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const v4h_ml am = *(const v4h_ml*)(S + L::H + (16 * t + jj) * 32 + 8 * q);
-                const v4f_ml z = {};
-                const v4f_ml ms = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, z, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; r++) accm[0][4 * t + r] = accm[0][4 * t + r] + dm[4 * t + r] * ms[r];
-            }
-#pragma unroll
-            for (int r = 0; r < 4 * RT; r++) asm volatile("" : "+v"(accm[0][r]));
-            __builtin_amdgcn_sched_barrier(0);
-        } else if constexpr (F::kMins) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                const uint32_t mwd = k < 2 ? sc.mn_lo : sc.mn_hi;
-                const _Float16 mA = (_Float16)(float)byte_of(mwd, 2 * (k & 1));
-                const _Float16 mB = (_Float16)(float)byte_of(mwd, 2 * (k & 1) + 1);
-                // B[kappa][col], kappa = 4 q + e: nonzero for q == k
-                const _Float16 zh = (_Float16)0.f;
-                const v4h_ml bm = q == k ? v4h_ml{mA, mA, mB, mB} : v4h_ml{zh, zh, zh, zh};
-#pragma unroll
-                for (int t = 0; t < RT; t++) {
-                    const v4h_ml am = *(const v4h_ml*)(S + L::H + (16 * t + jj) * 32 + 8 * q);
-                    const v4f_ml z = {};
-                    const v4f_ml ms = __builtin_amdgcn_mfma_f32_16x16x16f16(am, bm, z, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) accm[k][4 * t + r] = __builtin_fmaf(dm[4 * t + r], ms[r], accm[k][4 * t + r]);
-                }
-#pragma unroll
-                for (int r = 0; r < 4 * RT; r++) asm volatile("" : "+v"(accm[k][r]));
-                __builtin_amdgcn_sched_barrier(0);
-            }
         }
         __builtin_amdgcn_sched_barrier(0);
         if (b + 1 < nb) park(st[(b + 1) & 1]);
         lds_barrier();
     }
-    // hsum_f32_8 and hsum_f32_4 over the lane chains
+    // hsum_f32_8 over the lane chains
 #pragma unroll
-    for (int r = 0; r < 4 * RT; r++) {
+    for (int r = 0; r < 4; r++)
         v[r] = ((acc[0][r] + acc[4][r]) + (acc[2][r] + acc[6][r])) + ((acc[1][r] + acc[5][r]) + (acc[3][r] + acc[7][r]));
-        if constexpr (FMT == kQ5_K) v[r] = v[r] + accm[0][r];  // the mins scalar
-        else if constexpr (F::kMins) v[r] = v[r] + ((accm[0][r] + accm[2][r]) + (accm[1][r] + accm[3][r]));
-    }
 }
 
 // ---- up to 8 activation rows: two reference lanes per MFMA ------------------

@@ -102,7 +102,7 @@ hipError_t launch_moe_shared_combine(const float* x, const float* selector, cons
 // events (may be null): 4 hipEvent_t recorded before and between the launches.
 hipError_t launch_moe(const MoeParams& p, int gate_dtype, int down_dtype, hipStream_t s,
                       hipEvent_t const* events = nullptr);
-// The many-token path on int8 MFMA (iq_moe_prefill.hip).
+// The many-token path on MFMA (iq_moe_prefill.hip).
 bool moep_supported(const MoeParams& p, int gate_dtype, int down_dtype);
 hipError_t launch_moe_prefill(const MoeParams& p, int gate_dtype, int down_dtype, hipStream_t s,
                               hipEvent_t const* events);

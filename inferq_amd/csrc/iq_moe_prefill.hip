@@ -1,11 +1,11 @@
 // iq_moe_prefill.hip -- the MoE sublayer for many tokens (prefill widths),
 // grouped by expert (routed_grouped_by_expert, src/qwen/quantized_moe.rs:
-// 336-460), with the expert products on int8 MFMA in the reference's exact
+// 336-460), with the expert products on MFMA in the reference's exact
 // per-lane order: every token's output is bitwise what a one-token call
 // gives.
 //
 // The expert products are the exact lane-order MFMA tiles of
-// iq_mfma_lanes.h, so the bit pattern of every output matches the
+// iq_mfma_half.h (Q4_K, Q5_K) and iq_mfma_lanes.h (Q6_K), so the bit pattern of every output matches the
 // reference's per-lane FMA chains.
 //
 // Six launches per call:
@@ -319,7 +319,7 @@ __global__ __launch_bounds__(kMpThreads) void k_mp_group(MoeParams p) {
 
 // ------------------------------------------------------ expert products
 // Grid (column tiles, chunk bound).  A workgroup owns one chunk (kMpRows
-// grouped rows) and 64 weight rows (ml_product: wave w owns 16 of them and
+// grouped rows) and 64 weight rows (mh_product or ml_product: wave w owns 16 of them and
 // every 16-row tile of the chunk).  MODE 0: gate/up, weight rows i0 + 0..31 of
 // gate (waves 0, 1) and of up (waves 2, 3), A the chunk's tokens of x;
 // SwiGLU into act.  MODE 1: down, 64 hidden rows, A the chunk's act rows;
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(256) void k_mp_mm(MoeParams p) {
 #pragma unroll
         for (int r = 0; r < 4 * kMpRT; r++) v[r] = r < 4 ? vp[r] : 0.f;
     } else {
-        ml_product<FMT, kMpRT>(op, arow, brow, st, v);
+        ml_product(op, arow, brow, st, v);
     }
     auto out_row = [&](int r) { return pk ? (r < 4 ? 4 * (q & 1) + r : kMpRows) : 16 * (r >> 2) + 4 * q + (r & 3); };
     const bool writer = !pk || q < 2;  // pair-lane tiles: lane groups 2, 3 repeat 0, 1
