@@ -236,27 +236,6 @@ __device__ __forceinline__ Q4Dec q4_decode_lds(const uint8_t* b, int k) {
     return q4_decode(w, k);
 }
 
-// Q8_0: the 8 blocks of a unit at LDS address b (16-byte aligned).
-struct Q8Dec {
-    uint32_t q[8];
-    float d[8];
-};
-__device__ __forceinline__ Q8Dec q8_decode_lds(const uint8_t* b, int k) {
-    Q8Dec r;
-#pragma unroll
-    for (int c = 0; c < 8; c++) {
-        const uint8_t* blk = b + 34 * c;
-        if (c % 2 == 0) {  // window at 2 (mod 4)
-            const u32x2 v = *(const u32x2*)(blk + 4 * k);
-            r.q[c] = __builtin_amdgcn_alignbyte(v.y, v.x, 2);
-        } else {
-            r.q[c] = *(const uint32_t*)(blk + 2 + 4 * k);
-        }
-        r.d[c] = f16_to_f32(*(const uint16_t*)blk);
-    }
-    return r;
-}
-
 // ---- the kernel ----------------------------------------------------------------
 
 template <int FMT, int MT, int RPW, int NBUF, bool AMX = false>

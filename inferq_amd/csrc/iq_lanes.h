@@ -468,4 +468,25 @@ __device__ __forceinline__ void lanes_dot(const uint8_t* const (&wrow)[R], int n
     lanes_finish<FMT, MT, R>(acc, accm, out);
 }
 
+// Q8_0: the 8 blocks of a unit at LDS address b (16-byte aligned).
+struct Q8Dec {
+    uint32_t q[8];
+    float d[8];
+};
+__device__ __forceinline__ Q8Dec q8_decode_lds(const uint8_t* b, int k) {
+    Q8Dec r;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const uint8_t* blk = b + 34 * c;
+        if (c % 2 == 0) {  // window at 2 (mod 4)
+            const u32x2 v = *(const u32x2*)(blk + 4 * k);
+            r.q[c] = __builtin_amdgcn_alignbyte(v.y, v.x, 2);
+        } else {
+            r.q[c] = *(const uint32_t*)(blk + 2 + 4 * k);
+        }
+        r.d[c] = f16_to_f32(*(const uint16_t*)blk);
+    }
+    return r;
+}
+
 }  // namespace iq

@@ -95,6 +95,11 @@ hipError_t launch_moe_router(const MoeParams& p, hipStream_t s);
 // from theirs): act = SwiGLU(g, u) over n values, then out = residual +
 // (out + shared * sigmoid(x . selector)) for m tokens of width H.
 hipError_t launch_moe_swiglu(const float* g, const float* u, int64_t n, float* act, hipStream_t s);
+// All of it and the products of a Q8_0 shared expert, for few tokens (else
+// hipErrorNotSupported, nothing launched); act [m][I], sgate [m].
+hipError_t launch_moe_s8(const WeightView& gate, const WeightView& up, const WeightView& down, const float* x,
+                         const float* selector, const float* residual, int64_t m, float* act, float* sgate, float* out,
+                         hipStream_t s);
 hipError_t launch_moe_shared_combine(const float* x, const float* selector, const float* shared, const float* residual,
                                      int64_t m, int64_t H, float* out, hipStream_t s);
 

@@ -841,6 +841,152 @@ __global__ __launch_bounds__(256) void k_moe_shared_combine(const float* __restr
     }
 }
 
+// ---- the same for a Q8_0 shared expert and few tokens, in two launches ----
+//
+// A [512 x 2048] product of a few rows is all latency: gate, up, SwiGLU, down
+// and the combination took 23 us of a 42 us call of 2 tokens, five launches
+// of 3 to 6 us (now 9.6 of 29).  Here a workgroup takes one token and a few rows, quantises
+// the token's values itself while its weight rows (contiguous, 16 bytes a
+// lane) are in flight, and walks them in LDS; gate and up meet in LDS for
+// SwiGLU, and down's workgroups add the routed sum and the residual.  The
+// weights (3.3 MB) are read again for every token, from L2: a rising cost,
+// see kMoeS8Max.
+
+constexpr int kMoeS8Cols = 2048;  // widest hidden and intermediate size: a wave stages 8 rows in LDS
+// widest call (Q4_K / Q6_K experts, the whole layer, against the products of
+// their own launches): 1 token 24.2 / 36.9 us, 8: 54.6 / 71.3, 32: 138 / 146,
+// 48: 172 / 177, 64: 194 / 181
+constexpr int kMoeS8Max = 48;
+
+struct MoeS8 {
+    const uint8_t *gate, *up, *down;
+    const float *x, *selector, *residual;
+    int H, I;
+    float *act, *sgate, *out;
+};
+
+// LDS bytes between staged rows of nb blocks: an odd number of 32-byte steps
+// where it can be, so that 8 rows' dwords lie on distinct banks.
+__device__ __forceinline__ int s8_stride(int nb) {
+    const int rb = 34 * nb;
+    return (rb & 32) ? rb : rb + 32;
+}
+
+// One token's rows r0 .. r0 + 7 of a Q8_0 matrix of 32 nb columns: lane (slot,
+// k) returns row r0 + slot's product (hsum_f32_8, in every lane of the slot).
+// The workgroup's four waves call it together; x is quantised once, in
+// shared LDS.  PL: 16-byte loads a lane keeps in flight.
+template <int PL>
+__device__ __forceinline__ float s8_rows(const uint8_t* w, int64_t r0, int nb, const float* x, uint8_t* st,
+                                         uint32_t* s_q, float* s_d) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k = lane & 7, slot = lane >> 3;
+    const int gr = 34 * nb / 16, n16 = 8 * gr, stride = s8_stride(nb);  // nb a multiple of 8
+    const uint8_t* src = w + r0 * (34 * nb);
+    u32x4 v[PL];
+    auto issue = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < PL; i++) v[i] = *(const u32x4*)(src + 16 * (int64_t)min(i0 + lane + 64 * i, n16 - 1));
+    };
+    auto park = [&](int i0) {
+#pragma unroll
+        for (int i = 0; i < PL; i++) {
+            const int t = i0 + lane + 64 * i;
+            if (t < n16) {
+                const int r = t / gr;
+                *(u32x4a16*)(st + r * stride + 16 * (t - r * gr)) = u32x4a16{v[i].x, v[i].y, v[i].z, v[i].w};
+            }
+        }
+    };
+    const int ng = nb / 8;
+    f32x4 xv[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) xv[i] = q80_vals4_load(x, 32 * (int64_t)nb, min(wave + 4 * i, ng - 1));
+    issue(0);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const int g = wave + 4 * i;
+        const Q80Lane r = quant_q80_core(xv[i]);
+        if (g < ng) {
+            s_q[g * 64 + perm_dword(slot, k)] = r.packed;
+            if (k == 0) s_d[g * 8 + slot] = f16_to_f32(r.dh);
+        }
+    }
+    for (int i0 = 0; i0 < n16; i0 += 64 * PL) {
+        if (i0) issue(i0);
+        park(i0);
+    }
+    __syncthreads();
+    float acc = 0.f;
+    const uint8_t* row = st + slot * stride;
+#pragma unroll 2
+    for (int u = 0; u < ng; u++) {
+        const Q8Dec dec = q8_decode_lds(row + 272 * u, k);
+        const u32x4a16 a0 = *(const u32x4a16*)(s_q + u * 64 + 8 * k), a1 = *(const u32x4a16*)(s_q + u * 64 + 8 * k + 4);
+        const f32x4 d0 = *(const f32x4*)(s_d + 8 * u), d1 = *(const f32x4*)(s_d + 8 * u + 4);
+        const uint32_t av[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
+        const float yd[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+#pragma unroll
+        for (int c = 0; c < 8; c++) acc = __builtin_fmaf(dec.d[c] * yd[c], (float)sdot4(dec.q[c], av[c], 0), acc);
+    }
+    return hsum8(acc);
+}
+
+// Grid (I / 16 + 1, M): rows 16 b .. 16 b + 15 of gate (waves 0, 1) and of up
+// (waves 2, 3) and their SwiGLU; the last workgroup forms the token's gate.
+__global__ __launch_bounds__(256) void k_moe_s8_gate_up(MoeS8 a) {
+    __shared__ __align__(16) uint8_t st[4][8 * (kMoeS8Cols / 32 * 34 + 32)];
+    __shared__ __align__(16) uint32_t s_q[kMoeS8Cols / 4];
+    __shared__ __align__(16) float s_d[kMoeS8Cols / 32];
+    __shared__ float s_y[32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t t = blockIdx.y;
+    const float* x = a.x + t * a.H;
+    if ((int)blockIdx.x == a.I / 16) {  // whole workgroup
+        if (wave == 0) {
+            const float g = selector_gate(x, a.selector, a.H);
+            if (lane == 0) a.sgate[t] = g;
+        }
+        return;
+    }
+    const float y = s8_rows<17>(wave < 2 ? a.gate : a.up, 16 * (int64_t)blockIdx.x + 8 * (wave & 1), a.H / 32, x, st[wave],
+                                s_q, s_d);
+    if ((lane & 7) == 0) s_y[8 * wave + (lane >> 3)] = y;
+    __syncthreads();
+    if (threadIdx.x < 16) {
+        const float g = s_y[threadIdx.x];
+        a.act[t * a.I + 16 * (int64_t)blockIdx.x + threadIdx.x] = __fdiv_rn(g, 1.f + exp_f32(-g)) * s_y[16 + threadIdx.x];
+    }
+}
+
+// Grid (H / 32, M): down's rows, then as k_moe_shared_combine.
+__global__ __launch_bounds__(256) void k_moe_s8_down(MoeS8 a) {
+    __shared__ __align__(16) uint8_t st[4][8 * (kMoeS8Cols / 32 * 34 + 32)];
+    __shared__ __align__(16) uint32_t s_q[kMoeS8Cols / 4];
+    __shared__ __align__(16) float s_d[kMoeS8Cols / 32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t t = blockIdx.y, r0 = 32 * (int64_t)blockIdx.x + 8 * wave, n = t * a.H + r0 + (lane >> 3);
+    const float o = a.out[n], gate = a.sgate[t], res = a.residual ? a.residual[n] : 0.f;
+    const float y = s8_rows<5>(a.down, r0, a.I / 32, a.act + t * a.I, st[wave], s_q, s_d);
+    float v = o + y * gate;
+    if (a.residual) v = res + v;  // src/qwen/quantized_layer.rs:212
+    if ((lane & 7) == 0) a.out[n] = v;
+}
+
+hipError_t launch_moe_s8(const WeightView& gate, const WeightView& up, const WeightView& down, const float* x,
+                         const float* selector, const float* residual, int64_t m, float* act, float* sgate, float* out,
+                         hipStream_t s) {
+    const int64_t H = gate.cols, I = gate.rows;
+    if (m < 1 || m > kMoeS8Max || gate.dtype != kQ8_0 || down.dtype != kQ8_0 || H % 256 || I % 256 || H > kMoeS8Cols ||
+        I > kMoeS8Cols || (((uintptr_t)gate.w | (uintptr_t)up.w | (uintptr_t)down.w) & 15))
+        return hipErrorNotSupported;
+    const MoeS8 a = {gate.w, up.w, down.w, x, selector, residual, (int)H, (int)I, act, sgate, out};
+    hipLaunchKernelGGL(k_moe_s8_gate_up, dim3((unsigned)(I / 16 + 1), (unsigned)m), dim3(256), 0, s, a);
+    if (hipError_t e = hipGetLastError()) return e;
+    hipLaunchKernelGGL(k_moe_s8_down, dim3((unsigned)(H / 32), (unsigned)m), dim3(256), 0, s, a);
+    return hipGetLastError();
+}
+
+
 
 
 hipError_t launch_moe_swiglu(const float* g, const float* u, int64_t n, float* act, hipStream_t s) {

@@ -323,8 +323,13 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
         // the reference's shared path: down(SwiGLU(gate . x, up . x)), then
         // out = residual + (routed + shared * sigmoid(x . selector))
         const int64_t I = L->layer.I, H = L->layer.H;
-        e = launch_q8_swiglu(view_of(&L->sgate), view_of(&L->sup), view_of(&L->sdown), x, m, p.shared_g, p.shared_u,
-                             p.shared_out, p.shared_ws, s);
+        const WeightView sg = view_of(&L->sgate), su = view_of(&L->sup), sd = view_of(&L->sdown);
+        // few tokens of a Q8_0 expert: the combination and its gate (kept in
+        // shared_out) included
+        e = launch_moe_s8(sg, su, sd, x, L->selector, residual, m, p.shared_act, p.shared_out, out, s);
+        const bool combined = e == hipSuccess;
+        if (e == hipErrorNotSupported)
+            e = launch_q8_swiglu(sg, su, sd, x, m, p.shared_g, p.shared_u, p.shared_out, p.shared_ws, s);
         if (e != hipSuccess && e != hipErrorNotSupported) return hip_fail(e, "MoE shared expert launch");
         if (e == hipErrorNotSupported) {
             if (int rc = matmul_impl(&L->sgate, x, m, p.shared_g, p.shared_ws, p.shared_ws_bytes, IQ_PATH_AUTO, nullptr,
@@ -339,7 +344,7 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
                                      IQ_PATH_AUTO, nullptr, nullptr, s))
                 return rc;
         }
-        e = launch_moe_shared_combine(x, L->selector, p.shared_out, residual, m, H, out, s);
+        if (!combined) e = launch_moe_shared_combine(x, L->selector, p.shared_out, residual, m, H, out, s);
         if (e != hipSuccess) return hip_fail(e, "MoE shared combine launch");
     }
     L->last = p;

@@ -119,3 +119,35 @@ def test_q8_shared_expert_wide_equals_narrow(gpu, tokens, hidden, inter):
     for i in range(0, tokens, 8):
         m.forward_into(x[i:i + 8].contiguous(), lg[i:i + 8].contiguous(), narrow[i:i + 8])
     assert_bitexact(wide.cpu().numpy(), narrow.cpu().numpy(), f"{tokens} tokens")
+
+
+# widths of one and several 256-value groups a wave, the widest (2048) and one past it, which runs as single products
+@pytest.mark.parametrize("hidden,inter", [(256, 256), (768, 1280), (2048, 512), (512, 2048), (2304, 256)])
+def test_q8_shared_expert_few_tokens(gpu, hidden, inter):
+    """1, 5 and 48 tokens (two launches for the shared expert, combination and residual included) and 49 (its products
+    apart) give each token what a call of 70 tokens gives it, bit for bit, with a residual added."""
+    import torch
+
+    from inferq_amd import moe as M, synth as S
+
+    rng = np.random.default_rng([hidden, inter])
+    layer = S.random_moe_layer(hidden, inter, 8, S.Q4_K, S.Q6_K, rng)
+    for name, r, c in (("shared_gate", inter, hidden), ("shared_up", inter, hidden), ("shared_down", hidden, inter)):
+        layer[name] = S.random_matrix(S.Q8_0, r, c, rng)
+    t = {k: torch.from_numpy(v).to(gpu) for k, v in layer.items() if isinstance(v, np.ndarray)}
+    m = M.QuantizedMoeLayer(hidden, inter, 8, 2, S.Q4_K, S.Q6_K, t["gate"], t["up"], t["down"], t["shared_gate"],
+                            t["shared_up"], t["shared_down"], t["selector"], shared_gate_dtype=S.Q8_0,
+                            shared_down_dtype=S.Q8_0, router=torch.from_numpy(S.normal((8, hidden), rng)).to(gpu))
+    x, res = (torch.from_numpy(S.normal((70, hidden), rng)).to(gpu) for _ in range(2))
+    x[3] = 0.0
+    wide = torch.empty_like(x)
+    m.forward_x_into(x, wide, res)
+    for n in (1, 5, 48, 49):
+        for r in (res, None):
+            got = torch.full((n + 1, hidden), 7.0, device=gpu)
+            m.forward_x_into(x[70 - n:].contiguous(), got[:n], None if r is None else r[70 - n:].contiguous())
+            assert torch.all(got[n] == 7.0)
+            if r is not None:
+                assert_bitexact(got[:n].cpu().numpy(), wide[70 - n:].cpu().numpy(), f"{n} tokens")
+            else:
+                assert torch.allclose(got[:n] + res[70 - n:], wide[70 - n:], rtol=0, atol=0)  # res + v, one addition
