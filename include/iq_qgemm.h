@@ -156,7 +156,7 @@ int iq_matmul(iq_weight_t w, const float *x, int64_t m, float *y, iq_stream_t st
 int iq_matmul_via(iq_weight_t w, const float *x, int64_t m, float *y, int path, iq_stream_t stream);
 
 /* Size the library workspace of `stream` (current device) for calls of up
- * to m input rows of W through iq_matmul, iq_matmul_via and
+ * to m input rows of W through iq_matmul, iq_matmul_via and (m <= 65535)
  * iq_matmul_argmax, so that such calls can be captured into a graph
  * without an eager call first.  Not during capture.
  * Replaces: the reference's load-time allocation of the per-call buffers
@@ -171,8 +171,8 @@ int iq_matmul_reserve(iq_weight_t w, int64_t m, iq_stream_t stream);
  * No counterpart in the reference (its per-call buffers are Rust Vecs). */
 int iq_workspace_release(iq_stream_t stream);
 
-/* Device workspace bytes iq_matmul_ws needs for m input rows of W (any
- * path). */
+/* Device workspace bytes that serve every iq_matmul_ws call of up to m input
+ * rows of W (any path): never less for more rows. */
 size_t iq_matmul_workspace_size(iq_weight_t w, int64_t m);
 
 /* iq_matmul with a caller-provided device workspace (>= the size above). */
@@ -183,7 +183,7 @@ int iq_matmul_ws(iq_weight_t w, const float *x, int64_t m, float *y, void *works
  * array per GPU (iq_matmul_noalloc_max_bytes()), resolved once per device
  * at iq_init (or at the first call on a device) and held until the process
  * ends.  Calls whose workspace would exceed it fail with IQ_ERR_RANGE
- * before any launch (iq_matmul_workspace_size tells the need).  Results
+ * before any launch (iq_matmul_workspace_size bounds the need).  Results
  * are bitwise iq_matmul's.  Every call on one GPU shares that array, so
  * calls that overlap in time on one device (other streams or threads)
  * race; serialise them.  Safe under graph capture: no allocation, no

@@ -262,6 +262,15 @@ size_t matmul_ws_bytes(const iq_weight* w, int64_t m) {
     return std::max({a, p, d, q8_few_workspace(view_of(w), m)});
 }
 
+// The most any product of up to m rows needs: what a caller of narrower calls
+// too must hold.  The tile kernels' own needs fall where their plans change.
+size_t matmul_ws_upto(const iq_weight* w, int64_t m) {
+    if (float_dtype(w->dtype)) return 0;
+    const WeightView v = view_of(w);
+    return std::max({act_bytes(m, w->cols), prefill_workspace_upto(v, m), dense_mfma_workspace_upto(v, m),
+                     q8_few_workspace(v, m)});
+}
+
 // Greedy selection fused into the product (iq_matmul_argmax): 1 = one row
 // on the four-row-item GEMV, 2 = 2..8 rows on the pair-lane MFMA tile, 0 =
 // none (the product, then launch_argmax over its logits).
@@ -289,6 +298,18 @@ size_t argmax_call_bytes(const iq_weight* w, int64_t m) {
     const size_t fused = P ? ((P * 8 + 255) & ~(size_t)255) + ((P * 4 + 255) & ~(size_t)255) + matmul_ws_bytes(w, m)
                            : 0;
     return yb + (rest > fused ? rest : fused);
+}
+
+// The most any iq_matmul_argmax call of up to m rows needs (fused calls have
+// up to 8 rows).
+size_t argmax_call_upto(const iq_weight* w, int64_t m) {
+    const size_t yb = ((size_t)(m * w->rows) * 4 + 255) & ~(size_t)255;
+    size_t extra = (argmax_workspace_size(m, w->rows) + 255) & ~(size_t)255;
+    for (int64_t i = 1; i <= std::min<int64_t>(m, 8); i++) {
+        const size_t P = (size_t)(i * argmax_fused_parts(w, i));
+        extra = std::max(extra, ((P * 8 + 255) & ~(size_t)255) + ((P * 4 + 255) & ~(size_t)255));
+    }
+    return yb + extra + matmul_ws_upto(w, m);
 }
 
 // Kernel choice of a product (iq_matmul_via's path argument).  Every path
@@ -513,7 +534,7 @@ IQ_API int iq_matmul_reserve(iq_weight_t w, int64_t m, iq_stream_t stream) {
     if (m < 0) return fail(IQ_ERR_SHAPE, "negative input row count %lld", (long long)m);
     if (m == 0) return IQ_OK;
     // the widest of the entries that use the stream's workspace for W
-    const size_t need = std::max(matmul_ws_bytes(w, m), m <= 65535 ? argmax_call_bytes(w, m) : 0);
+    const size_t need = std::max(matmul_ws_upto(w, m), m <= 65535 ? argmax_call_upto(w, m) : 0);
     WsLease lease;
     return lease.acquire(need, (hipStream_t)stream);
 }
@@ -522,7 +543,7 @@ IQ_API int iq_workspace_release(iq_stream_t stream) { return release_workspace((
 
 IQ_API size_t iq_matmul_workspace_size(iq_weight_t w, int64_t m) {
     if (!w || m <= 0) return 0;
-    return matmul_ws_bytes(w, m);
+    return matmul_ws_upto(w, m);
 }
 
 IQ_API int iq_matmul_ws(iq_weight_t w, const float* x, int64_t m, float* y, void* workspace_ptr,

@@ -51,6 +51,7 @@ int check_weight(const iq_weight* w);
 // y = x . W^T through the dispatch (or a fixed path), with the caller's
 // workspace when ws is not null (ws_bytes >= matmul_ws_bytes(w, m)).
 size_t matmul_ws_bytes(const iq_weight* w, int64_t m);
+size_t matmul_ws_upto(const iq_weight* w, int64_t m);  // what any call of up to m rows needs
 int matmul_impl(const iq_weight* w, const float* x, int64_t m, float* y, void* ws, size_t ws_bytes, int path,
                 int32_t* isum, int32_t* msum, hipStream_t s);
 WeightView view_of(const iq_weight* w);

@@ -268,13 +268,16 @@ DmPlan dm_plan(const WeightView& w, int64_t m) {
     return P;
 }
 
-// Rows of one pass: as many as 16 MiB of workspace hold (3912 of width
-// 2048), the call's rows spread evenly.  A wider call runs pass by pass (rows
-// are independent), so that its workspace does not outgrow what it was with
-// int8 activations.
-int64_t dm_pass_rows(const WeightView& w, int64_t m) {
+// Rows of the widest pass: as many as 16 MiB of workspace hold (3826 of
+// width 2048), what iq_matmul_noalloc has.  A wider call runs pass by pass
+// (rows are independent), its rows spread evenly.
+int64_t dm_max_pass_rows(const WeightView& w) {
     const int64_t per_row = w.cols / 256 * (kMhBlock + 36);
-    const int64_t most = std::max<int64_t>((((int64_t)16 << 20) - 1024) / per_row, 1), passes = (m + most - 1) / most;
+    return std::max<int64_t>((((int64_t)16 << 20) - 1024) / per_row, 1);
+}
+
+int64_t dm_pass_rows(const WeightView& w, int64_t m) {
+    const int64_t most = dm_max_pass_rows(w), passes = (m + most - 1) / most;
     return (m + passes - 1) / passes;
 }
 
@@ -359,6 +362,11 @@ bool dense_mfma_supported(const WeightView& w, int64_t m) {
 
 size_t dense_mfma_workspace_any(const WeightView& w, int64_t m) {
     return dm_layout_ok(w) && dm_rows_ok(w, m) ? dm_plan(w, dm_pass_rows(w, m)).total() : 0;
+}
+
+// A call just past the widest pass needs about half of that pass's bytes.
+size_t dense_mfma_workspace_upto(const WeightView& w, int64_t m) {
+    return m >= 1 && dm_layout_ok(w) ? dm_plan(w, std::min(m, dm_max_pass_rows(w))).total() : 0;
 }
 
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,

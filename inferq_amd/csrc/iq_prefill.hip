@@ -19,6 +19,8 @@
 // such tiles take 32 x 64 tiles (4 waves, two row tiles each) and, only if
 // those are still too few, a split over K, with partial tiles summed in a
 // fixed order by a second pass.
+#include <algorithm>
+
 #include "iq_lanes.h"
 #include "iq_pf_q4k.h"
 #include "iq_quant.h"
@@ -41,6 +43,8 @@ namespace {
 constexpr int kPfRows = 64, kPfCols = 128;      // large calls
 constexpr int kPfRowsS = 32, kPfColsS = 64;     // calls with fewer than 256 large tiles
 constexpr int kPfMinTiles = 256;
+constexpr int kPfMaxSplits = 8;
+constexpr int64_t kPfMaxRows = 1 << 20;
 
 // ---- activation quantisation --------------------------------------------------
 // Q8K (bit-exact from_float) into the layouts the MFMA kernel reads:
@@ -271,7 +275,7 @@ PfPlan plan(const WeightView& w, int64_t m) {
     P.mp = (int)((m + P.rows - 1) / P.rows * P.rows);
     const int64_t tiles = ((w.rows + P.cols - 1) / P.cols) * (P.mp / P.rows);  // real tiles (padding aside)
     int splits = 1;
-    while (tiles * splits < kPfMinTiles && splits * 2 <= P.nb && splits < 8) splits *= 2;
+    while (tiles * splits < kPfMinTiles && splits * 2 <= P.nb && splits < kPfMaxSplits) splits *= 2;
     P.bps = (P.nb + splits - 1) / splits;
     P.splits = (P.nb + P.bps - 1) / P.bps;
     P.q_bytes = align256((size_t)P.mp * P.nb * 256);
@@ -284,10 +288,24 @@ PfPlan plan(const WeightView& w, int64_t m) {
 }  // namespace
 
 bool prefill_supported(const WeightView& w, int64_t m) {
-    return w.dtype == kQ4_K && m >= kPrefillMinRows && w.cols % 256 == 0 && w.rows >= 1 && m <= (1 << 20);
+    return w.dtype == kQ4_K && m >= kPrefillMinRows && w.cols % 256 == 0 && w.rows >= 1 && m <= kPfMaxRows;
 }
 
 size_t prefill_workspace_size(const WeightView& w, int64_t m) { return prefill_supported(w, m) ? plan(w, m).total() : 0; }
+
+// More rows need fewer splits, so the need falls where their number does:
+// besides m, the last row count of each number of splits (their tiles stay
+// under 2 kPfMinTiles / splits).
+size_t prefill_workspace_upto(const WeightView& w, int64_t m) {
+    m = std::min<int64_t>(m, kPfMaxRows);
+    size_t most = prefill_workspace_size(w, m);
+    const int64_t col_tiles = (w.rows + kPfColsS - 1) / kPfColsS;
+    for (int splits = 2; splits <= kPfMaxSplits; splits *= 2) {
+        const int64_t last = (2 * kPfMinTiles / splits - 1) / col_tiles * kPfRowsS;
+        most = std::max(most, prefill_workspace_size(w, std::min(m, last)));
+    }
+    return most;
+}
 
 hipError_t launch_prefill(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
                           void* ws, int32_t* dbg_isum, int32_t* dbg_msum, hipStream_t s) {
