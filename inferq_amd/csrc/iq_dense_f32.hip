@@ -10,6 +10,8 @@
 // turn, then the 64 lanes meet in a butterfly (xor 32, 16, ..., 1).  BF16
 // weights widen to f32 exactly first.  Every pair is formed the same way at
 // any row count.
+#include <type_traits>
+
 #include "iq_device.h"
 #include "iq_internal.h"
 
@@ -25,29 +27,48 @@ __device__ __forceinline__ float float_w(const uint8_t* w, int64_t i) {
 
 // Few pairs: one wave per (weight row, input row), grid (n, m).  Latency
 // bound: a 2048-wide row's 32 loads of each operand are in flight at once
-// (one round trip).  A wave that took eight input rows in turn, eight values
-// at a time, made 4 x 8 dependent round trips: router [256 x 2048] at 8 rows
-// 18.5 -> 3.5 us, BF16 [64 x 2048] at 8 rows 14.4 -> 2.6 us.
+// (one round trip), what is left of a row goes in passes of 16 and 8 steps and
+// one cut short at its end.  A wave that took eight input rows in turn, eight
+// values at a time, made 4 x 8 dependent round trips: router [256 x 2048] at
+// 8 rows 18.5 -> 3.5 us, BF16 [64 x 2048] at 8 rows 14.4 -> 2.6 us; single
+// steps at the end of a row: [2048 x 1024] at 4 rows 6.6 against 4.8 us.
 template <bool BF16>
 __global__ __launch_bounds__(64) void k_float_pair(const uint8_t* __restrict__ w, int64_t k,
                                                    const float* __restrict__ x, int64_t ldx, float* __restrict__ y,
                                                    int64_t ldy) {
-    constexpr int U = 32;
     const int lane = threadIdx.x;
-    const int64_t row = blockIdx.x, t = blockIdx.y, w0 = row * k;
+    const int64_t row = blockIdx.x, t = blockIdx.y;
+    const uint8_t* wr = w + row * k * (BF16 ? 2 : 4);
     const float* xr = x + t * ldx;
     float part = 0.f;
-    int64_t h = lane;
-    for (; h + 64 * (U - 1) < k; h += 64 * U) {
+    // U steps of the chain from value h on; CUT: the row's last ones, those
+    // past its end on its last value and left out
+    int64_t h = 0;
+    auto pass = [&](auto U_, auto CUT_) {
+        constexpr int U = U_;
+        constexpr bool CUT = CUT_;
+        const int left = CUT ? (int)(k - h) : 0;
+        auto at = [&](int j) { return CUT ? min(lane + 64 * j, left - 1) : lane + 64 * j; };
+        const uint8_t* wh = wr + h * (BF16 ? 2 : 4);
         float rv[U], xv[U];
 #pragma unroll
-        for (int j = 0; j < U; j++) rv[j] = float_w<BF16>(w, w0 + h + 64 * j);
+        for (int j = 0; j < U; j++) rv[j] = float_w<BF16>(wh, at(j));
 #pragma unroll
-        for (int j = 0; j < U; j++) xv[j] = xr[h + 64 * j];
+        for (int j = 0; j < U; j++) xv[j] = xr[h + at(j)];
 #pragma unroll
-        for (int j = 0; j < U; j++) part = part + xv[j] * rv[j];
-    }
-    for (; h < k; h += 64) part = part + xr[h] * float_w<BF16>(w, w0 + h);
+        for (int j = 0; j < U; j++) {
+            const float v = part + xv[j] * rv[j];
+            part = !CUT || lane + 64 * j < left ? v : part;
+        }
+        h += 64 * U;
+    };
+    using std::integral_constant;
+    while (k - h >= 64 * 32) pass(integral_constant<int, 32>{}, std::false_type{});
+    if (k - h >= 64 * 16) pass(integral_constant<int, 16>{}, std::false_type{});
+    if (k - h >= 64 * 8) pass(integral_constant<int, 8>{}, std::false_type{});
+    if (k - h > 64 * 4) pass(integral_constant<int, 8>{}, std::true_type{});
+    else if (k - h > 64) pass(integral_constant<int, 4>{}, std::true_type{});
+    else if (k - h > 0) pass(integral_constant<int, 1>{}, std::true_type{});
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) part = part + __shfl_xor(part, off);
     if (lane == 0) y[t * ldy + row] = part;
