@@ -25,22 +25,26 @@ __device__ __forceinline__ float float_w(const uint8_t* w, int64_t i) {
     else return ((const float*)w)[i];
 }
 
-// Few pairs: one wave per (weight row, input row), grid (n, m).  Latency
-// bound: a 2048-wide row's 32 loads of each operand are in flight at once
-// (one round trip), what is left of a row goes in passes of 16 and 8 steps and
-// one cut short at its end.  A wave that took eight input rows in turn, eight
-// values at a time, made 4 x 8 dependent round trips: router [256 x 2048] at
-// 8 rows 18.5 -> 3.5 us, BF16 [64 x 2048] at 8 rows 14.4 -> 2.6 us; single
-// steps at the end of a row: [2048 x 1024] at 4 rows 6.6 against 4.8 us.
-template <bool BF16>
+// Few pairs, or few input rows: one wave per weight row and TT input rows,
+// grid (n, ceil(m / TT)).  Latency bound: a 2048-wide row's 32 loads of each
+// operand are in flight at once (one round trip), what is left of a row goes
+// in passes of 16 and 8 steps and one cut short at its end.  A wave that took
+// eight input rows in turn, eight values at a time, made 4 x 8 dependent round
+// trips: router [256 x 2048] at 8 rows 18.5 -> 3.5 us, BF16 [64 x 2048] at 8
+// rows 14.4 -> 2.6 us; single steps at the end of a row: [2048 x 1024] at 4
+// rows 6.6 against 4.8 us.
+template <bool BF16, int TT, int UM>
 __global__ __launch_bounds__(64) void k_float_pair(const uint8_t* __restrict__ w, int64_t k,
-                                                   const float* __restrict__ x, int64_t ldx, float* __restrict__ y,
-                                                   int64_t ldy) {
+                                                   const float* __restrict__ x, int64_t ldx, int m,
+                                                   float* __restrict__ y, int64_t ldy) {
     const int lane = threadIdx.x;
-    const int64_t row = blockIdx.x, t = blockIdx.y;
+    const int64_t row = blockIdx.x;
+    const int t0 = (int)blockIdx.y * TT, nt = min(TT, m - t0);
     const uint8_t* wr = w + row * k * (BF16 ? 2 : 4);
-    const float* xr = x + t * ldx;
-    float part = 0.f;
+    const float* xr = x + (int64_t)t0 * ldx;
+    float part[TT];
+#pragma unroll
+    for (int i = 0; i < TT; i++) part[i] = 0.f;
     // U steps of the chain from value h on; CUT: the row's last ones, those
     // past its end on its last value and left out
     int64_t h = 0;
@@ -54,24 +58,33 @@ __global__ __launch_bounds__(64) void k_float_pair(const uint8_t* __restrict__ w
 #pragma unroll
         for (int j = 0; j < U; j++) rv[j] = float_w<BF16>(wh, at(j));
 #pragma unroll
-        for (int j = 0; j < U; j++) xv[j] = xr[h + at(j)];
+        for (int i = 0; i < TT; i++) {
+            if (TT > 1 && i >= nt) break;  // uniform
+            const float* xh = xr + i * ldx + h;
 #pragma unroll
-        for (int j = 0; j < U; j++) {
-            const float v = part + xv[j] * rv[j];
-            part = !CUT || lane + 64 * j < left ? v : part;
+            for (int j = 0; j < U; j++) xv[j] = xh[at(j)];
+#pragma unroll
+            for (int j = 0; j < U; j++) {
+                const float v = part[i] + xv[j] * rv[j];
+                part[i] = !CUT || lane + 64 * j < left ? v : part[i];
+            }
         }
         h += 64 * U;
     };
     using std::integral_constant;
-    while (k - h >= 64 * 32) pass(integral_constant<int, 32>{}, std::false_type{});
-    if (k - h >= 64 * 16) pass(integral_constant<int, 16>{}, std::false_type{});
-    if (k - h >= 64 * 8) pass(integral_constant<int, 8>{}, std::false_type{});
+    while (k - h >= 64 * UM) pass(integral_constant<int, UM>{}, std::false_type{});
+    if (UM > 16 && k - h >= 64 * 16) pass(integral_constant<int, 16>{}, std::false_type{});
+    if (UM > 8 && k - h >= 64 * 8) pass(integral_constant<int, 8>{}, std::false_type{});
     if (k - h > 64 * 4) pass(integral_constant<int, 8>{}, std::true_type{});
     else if (k - h > 64) pass(integral_constant<int, 4>{}, std::true_type{});
     else if (k - h > 0) pass(integral_constant<int, 1>{}, std::true_type{});
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) part = part + __shfl_xor(part, off);
-    if (lane == 0) y[t * ldy + row] = part;
+    for (int i = 0; i < TT; i++) {
+        float v = part[i];
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) v = v + __shfl_xor(v, off);
+        if (lane == 0 && (TT == 1 || i < nt)) y[(t0 + i) * ldy + row] = v;
+    }
 }
 
 // Butterfly step of N values per lane at distance OFF, halving them: the
@@ -215,8 +228,23 @@ hipError_t launch_tile(const WeightView& w, const float* x, int64_t ldx, int64_t
     return hipGetLastError();
 }
 
+template <bool BF16, int TT, int UM>
+hipError_t launch_pair(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, hipStream_t s) {
+    const dim3 grid((unsigned)w.rows, (unsigned)((m + TT - 1) / TT));
+    hipLaunchKernelGGL((k_float_pair<BF16, TT, UM>), grid, dim3(64), 0, s, w.w, w.cols, x, ldx, (int)m, y, ldy);
+    return hipGetLastError();
+}
+
 // Up to 8192 pairs one wave each ([256 x 2048] at 32 / 64 rows: pairs 6.5 /
-// 10.3 us, tiles 7.0 / 7.4).  Tiles of 4 x 4 pairs a wave with 512 values a
+// 10.3 us, tiles 7.0 / 7.4).  Tall matrices at one to three rows stream, a
+// wave per weight row for all of them, 16 steps at a time where that leaves
+// more waves in flight: a tile multiplies eight input rows whatever the call
+// has.  us, streamed / tile: BF16 [32000 x 2048] at 1 / 2 / 3 rows 20.4 / 38.6,
+// 25.4 / 38.6, 33.3 / 38.7 (4 rows: 40.9 / 38.7), F32 [8200 x 2048] 12.0 / 18.4,
+// 12.9 / 18.8, 13.9 / 19.4; two rows against a wave each [2048 x 2048] 4.8 /
+// 4.8, [4096 x 2048] 6.0 / 6.5.  Three rows past 256 MiB, out of the Infinity
+// Cache's reach, and of 512 columns take the tile: BF16 [64000 x 4096] 182 /
+// 152, [32000 x 512] 14.1 / 13.0.  Tiles of 4 x 4 pairs a wave with 512 values a
 // stage while they leave at most two workgroups per CU, whose barriers and
 // round trips then cost more than the LDS they take ([64 x 2048] at 512 rows
 // 9.4 against 10.3 us with 256; [256 x 2048] at 256 rows 14.6 against 12.4);
@@ -225,11 +253,11 @@ hipError_t launch_tile(const WeightView& w, const float* x, int64_t ldx, int64_t
 template <bool BF16>
 hipError_t launch_bf(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy, hipStream_t s) {
     const int64_t tiles = ((w.rows + 7) / 8) * ((m + 7) / 8), wide = ((w.rows + 15) / 16) * ((m + 7) / 8);
-    if (w.rows * m <= 8192) {
-        hipLaunchKernelGGL((k_float_pair<BF16>), dim3((unsigned)w.rows, (unsigned)m), dim3(64), 0, s, w.w, w.cols, x, ldx, y,
-                           ldy);
-        return hipGetLastError();
-    }
+    const bool few = m <= 3 && w.rows < (int64_t)1 << 26;  // a launch has at most 2^32 threads
+    if (few && m == 2 && w.rows > 2048) return launch_pair<BF16, 2, 16>(w, x, ldx, m, y, ldy, s);
+    if ((few && m == 1) || w.rows * m <= 8192) return launch_pair<BF16, 1, 32>(w, x, ldx, m, y, ldy, s);
+    if (few && m == 3 && w.cols >= 1024 && w.rows * w.row_bytes <= (int64_t)256 << 20)
+        return launch_pair<BF16, 3, 16>(w, x, ldx, m, y, ldy, s);
     if (tiles <= 512) return launch_tile<BF16, 4, 4, 8>(w, x, ldx, m, y, ldy, s);
     if (wide < 1024) return launch_tile<BF16, 4, 4, 4>(w, x, ldx, m, y, ldy, s);
     return launch_tile<BF16, 8, 4, 4>(w, x, ldx, m, y, ldy, s);
