@@ -8,6 +8,12 @@ namespace iq {
 constexpr int kMoeMaxExperts = 512;   // routed experts per layer
 constexpr int kMoeMaxTopK = 16;       // experts per token
 constexpr int kMoeMaxAssign = 4096;   // tokens * top_k per call
+// expert x 32-token words of a grouped call: six bytes of LDS each (a mask and
+// a count), 48 KiB beside the grouping kernel's 2.5 KiB of its own, under the
+// 64 KiB a launch may ask for without raising the kernel's limit
+constexpr int kMoeMaskWords = 8192;
+constexpr int kMoeMaskWordBytes = 6;
+static_assert(kMoeMaskWords * kMoeMaskWordBytes + 4096 <= 65536, "grouping kernel's LDS");
 constexpr int kMoePrefillMinTokens = 17;  // the MFMA path serves calls of this many tokens or more
 
 struct MoeParams {

@@ -129,13 +129,14 @@ size_t carve(iq_moe* L, int m, uint8_t* base, MoeParams* p) {
 
 // Tokens one set of launches serves: the grouping kernels keep every
 // (token, route) pair of a call on chip (kMoeMaxAssign of them), and the
-// many-token path keeps a bitmask of tokens per expert in 32 KiB of LDS.
+// many-token path keeps a bitmask of tokens per expert (kMoeMaskWords words)
+// in LDS.
 // A wider call runs as consecutive slices of this many tokens; every
 // token's output is independent of the others in its call, so the slices
 // give the same bits as one call would.
 int slice_tokens(const iq_moe* L) {
     const int64_t by_assign = kMoeMaxAssign / L->layer.K;
-    const int64_t by_mask = 32 * (8192 / std::max<int64_t>(L->layer.E, 1));
+    const int64_t by_mask = 32 * (kMoeMaskWords / std::max<int64_t>(L->layer.E, 1));
     return (int)std::max<int64_t>(1, std::min(by_assign, by_mask));
 }
 

@@ -184,7 +184,8 @@ __device__ __forceinline__ void block_scan(int (&v)[N], int* s_tmp /* [N][17] */
 // the long ones go first and the short ones fill the last round (the order
 // changes which rows share a launch round, never a result).
 __global__ __launch_bounds__(kMpThreads) void k_mp_group(MoeParams p) {
-    extern __shared__ uint32_t s_mask[];  // [mw][E] token bitmasks, then [mw][E] tokens in the words before
+    // [mw][E] token bitmasks, then [mw][E] tokens in the words before (16 bits: at most kMoeMaxAssign)
+    extern __shared__ uint32_t s_mask[];
     __shared__ int s_start[kMoeMaxExperts];
     __shared__ int s_tmp[4 * 17];
     __shared__ int s_pcnt[kMpRows], s_pbase[kMpRows], s_pnext[kMpRows];  // partial chunks by rows
@@ -209,11 +210,11 @@ __global__ __launch_bounds__(kMpThreads) void k_mp_group(MoeParams p) {
         }
     }
     __syncthreads();
-    uint32_t* s_pre = s_mask + E * mw;
+    uint16_t* s_pre = (uint16_t*)(s_mask + E * mw);
     int cnt = 0;
     if (tid < E)
         for (int w = 0; w < mw; w++) {
-            s_pre[w * E + tid] = (uint32_t)cnt;
+            s_pre[w * E + tid] = (uint16_t)cnt;
             cnt += __popc(s_mask[w * E + tid]);
         }
     const int nfull = cnt / kMpRows, rpart = cnt % kMpRows;  // full chunks, rows of the partial one (0: none)
@@ -731,7 +732,7 @@ hipError_t launch_p(const MoeParams& p, hipStream_t s, hipEvent_t const* ev) {
     const int64_t qw = (int64_t)M * nbH;
     hipLaunchKernelGGL((k_mp_route<kMpHalf<GFMT>>), dim3((unsigned)(nr + (qw + 15) / 16)), dim3(kMpThreads), 0, s, p);
     if (hipError_t e = hipGetLastError()) return e;
-    const size_t mask_bytes = (size_t)p.E * ((M + 31) / 32) * 8;
+    const size_t mask_bytes = (size_t)p.E * ((M + 31) / 32) * kMoeMaskWordBytes;
     hipLaunchKernelGGL(k_mp_group, dim3(1), dim3(kMpThreads), mask_bytes, s, p);
     if (hipError_t e = hipGetLastError()) return e;
     if (ev) (void)hipEventRecord(ev[1], s);
@@ -781,7 +782,7 @@ bool moep_supported(const MoeParams& p, int gfmt, int dfmt) {
                          al(p.residual, 16);  // k_mp_combine moves four floats at a time
     return kq && aligned && p.M >= kMoePrefillMinTokens && p.H % 256 == 0 && p.I % 256 == 0 && p.E <= kMoeMaxExperts &&
            p.K <= kMoeMaxTopK && p.g_row_bytes % 4 == 0 && p.d_row_bytes % 4 == 0 &&
-           (int64_t)p.E * ((p.M + 31) / 32) * 4 <= 32768 && p.xhs != nullptr && p.chunk_group != nullptr &&
+           (int64_t)p.E * ((p.M + 31) / 32) <= kMoeMaskWords && p.xhs != nullptr && p.chunk_group != nullptr &&
            p.xh != nullptr && p.ah != nullptr && ((dfmt != kQ4_K && dfmt != kQ5_K) || p.ahs != nullptr);
 }
 
