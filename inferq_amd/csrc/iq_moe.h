@@ -58,8 +58,8 @@ struct MoeParams {
     // MFMA (prefill) path
     _Float16* xhs = nullptr;        // [M][H/256][16] 16-value sums of quantised x
     _Float16* ahs = nullptr;        // [P][I/256][16] the same of quantised act
-    int8_t* xh = nullptr;           // [M][H/256][512] quantised x as f16 (iq_mfma_half.h), for Q4_K / Q5_K gate and up
-    int8_t* ah = nullptr;           // [P][I/256][512] quantised act as f16, for Q4_K / Q5_K down
+    int8_t* xh = nullptr;           // [M][H/256][512] quantised x as f16 where moe_half(gate format), else null
+    int8_t* ah = nullptr;           // [P][I/256][512] quantised act as f16 where moe_half(down format), else null
     int32_t* chunk_group = nullptr;  // [max_chunks] group of each chunk of rows
     int32_t* chunk_r0 = nullptr;     // [max_chunks] first row of the chunk in its group
     int max_chunks = 0;
@@ -83,6 +83,10 @@ struct MoeParams {
     int32_t* experts_out = nullptr;  // [M][K]
     float* weights_out = nullptr;    // [M][K]
 };
+
+// Expert formats whose grouped products run on f16 MFMA (iq_mfma_half.h) and
+// read the f16 activations xh (gate, up) or ah (down).
+constexpr bool moe_half(int fmt) { return fmt == kQ4_K || fmt == kQ5_K; }
 
 constexpr int kMpRows = 16;  // grouped rows per chunk of the exact expert products
 #ifndef IQ_MP_TILE_ROWS

@@ -71,8 +71,8 @@ size_t carve(iq_moe* L, int m, uint8_t* base, MoeParams* p) {
     const int maxtch = moep_max_chunks(m, K, L->layer.E, kMpTileRows);
     uint8_t* xhs = take(m * ngH * 32);
     uint8_t* ahs = take(P * ngI * 32);
-    uint8_t* xh = take(m * ngH * 512);
-    uint8_t* ah = take(P * ngI * 512);
+    uint8_t* xh = moe_half(L->gfmt) ? take(m * ngH * 512) : nullptr;
+    uint8_t* ah = moe_half(L->dfmt) ? take(P * ngI * 512) : nullptr;
     uint8_t* chg = take((size_t)maxch * 4);
     uint8_t* chr = take((size_t)maxch * 4);
     uint8_t* tchg = take((size_t)maxtch * 4);

@@ -56,7 +56,7 @@ static_assert(kMpRows == 16 * kMpRT, "chunk rows");
 // launch of 512 tokens 78 -> 70.  Q6_K keeps the
 // int8 tiles, which at 16 rows decode it faster.
 template <int FMT>
-constexpr bool kMpHalf = FMT == kQ4_K || FMT == kQ5_K;
+constexpr bool kMpHalf = moe_half(FMT);
 constexpr int kMpTileRT = kMpTileRows / 16;  // 16-row tiles per chunk of the tile-order down
 #ifndef IQ_MP_RES_CT
 #define IQ_MP_RES_CT 2
@@ -783,7 +783,7 @@ bool moep_supported(const MoeParams& p, int gfmt, int dfmt) {
     return kq && aligned && p.M >= kMoePrefillMinTokens && p.H % 256 == 0 && p.I % 256 == 0 && p.E <= kMoeMaxExperts &&
            p.K <= kMoeMaxTopK && p.g_row_bytes % 4 == 0 && p.d_row_bytes % 4 == 0 &&
            (int64_t)p.E * ((p.M + 31) / 32) <= kMoeMaskWords && p.xhs != nullptr && p.chunk_group != nullptr &&
-           p.xh != nullptr && p.ah != nullptr && ((dfmt != kQ4_K && dfmt != kQ5_K) || p.ahs != nullptr);
+           (!moe_half(gfmt) || p.xh != nullptr) && (!moe_half(dfmt) || (p.ah != nullptr && p.ahs != nullptr));
 }
 
 hipError_t launch_moe_prefill(const MoeParams& p, int gfmt, int dfmt, hipStream_t s, hipEvent_t const* ev) {
