@@ -384,12 +384,13 @@ constexpr size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 // Measured, tile / GEMV: [8192 x 2048] at 9 / 16 rows 21.6 / 20.8 and 21.6 /
 // 27.1 us, [12288 x 2048] at 9 rows 22 / 32, [4096 x 4096] at 16 rows 37 / 28,
 // [8192 x 4096] at 16 rows 40 / 43, [512 x 2048] at 63 rows 20 / 12, [2048 x
-// 1024] at 63 rows 13 / 16.
+// 1024] at 32 / 63 rows 13.2 / 11.3 and 13 / 16, [4096 x 1024] at 16 / 20 rows
+// 12.0 / 11.3 and 13.2 / 17.0 (the GEMV's workgroups fill its last round).
 bool q8_tile_supported(const WeightView& w, int64_t m) {
     if (w.dtype != kQ8_0 || m < 9 || m > (int64_t)1 << 20 || w.rows < 1 || w.cols % (32 * kQtCB) != 0 ||
         ((uintptr_t)w.w & 3) != 0)
         return false;
-    return !gemv_supported(w, m) || (double)(w.rows * w.row_bytes) * (double)m / 8 > 1e6 * (0.4 * (double)(w.cols / 32) - 4);
+    return !gemv_supported(w, m) || (double)(w.rows * w.row_bytes) * (double)m / 8 > 1e6 * (0.4 * (double)(w.cols / 32) - 3.8);
 }
 
 namespace {
@@ -470,14 +471,18 @@ bool qf_shape(const WeightView& w) {
 // us: [2048 x 4096] at 6 / 7 rows 14.9 / 14.5 and 14.8 / 17.2, [4096 x 4096]
 // at 3 / 4 rows 17.0 / 15.0 and 17.1 / 18.1, [4096 x 2048] at 4 / 5 rows 11.3
 // / 11.0 and 11.4 / 14.5, [2048 x 1024] at 8 rows 7.6 / 7.5, [8192 x 1024] at
-// 5 rows 9.4 / 11.5.  Past 16384 rows the GEMV's waves fill the chip and it
-// reads the matrix at a better rate: [16000 x 2048] at 3 rows 19.4 / 24.9,
-// [24576 x 2048] at 4 rows 24.3 / 22.1, [32000 x 2048] at 4 / 6 rows 30.9 /
-// 29.1 and 29.1 / 34.0, [248320 x 2048] at 6 / 8 rows 177 / 163 and 177 / 199.
+// 5 rows 9.4 / 11.5.  From 16384 rows the GEMV's waves fill the chip and it
+// reads the matrix at a better rate: [16000 x 2048] at 3 rows 18.1 / 23.3,
+// [16384 x 2048] at 3 / 4 / 5 rows 18.4 / 14.8, 18.7 / 17.7 and 18.8 / 21.7
+// ([16384 x 1024] at 3 / 4 rows 11.8 / 12.0 and 12.1 / 13.5), [24576 x 2048] at
+// 4 / 5 / 6 rows 24.4 / 20.9, 24.6 / 25.2 and 24.8 / 27.2, [32000 x 2048] at 4
+// / 6 rows 30.9 / 29.1 and 29.1 / 34.0, [248320 x 2048] at 6 / 8 rows 177 / 163
+// and 177 / 199.
 // Rows of 6144: 20.4 / 17.9 at 8 rows, so not taken.
 bool q8_few_supported(const WeightView& w, int64_t m) {
     if (m < 3 || m > 8 || !qf_shape(w)) return false;
-    return m >= (w.rows <= 16384 ? 3 : w.rows <= 65536 ? 6 : 8) && w.rows * m * (w.cols / 32 + 64) >= 2500000;
+    const int64_t least = w.rows < 16384 ? 3 : w.rows < 24576 ? (w.cols <= 1024 ? 4 : 5) : w.rows <= 65536 ? 6 : 8;
+    return m >= least && w.rows * m * (w.cols / 32 + 64) >= 2500000;
 }
 
 size_t q8_few_workspace(const WeightView& w, int64_t m) {

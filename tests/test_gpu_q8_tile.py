@@ -55,6 +55,22 @@ def test_few_rows_bitwise(gpu, oracle, rows, cols, m):
     assert_bitexact(out[:m].cpu().numpy(), oracle.matmul(S.Q8_0, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
 
 
+# the lines of the rules, the tile on one side and the GEMV on the other
+@pytest.mark.parametrize("rows,cols,m", [(16383, 1024, 3), (16384, 1024, 4), (16384, 2048, 4), (16384, 2048, 5),
+                                         (24575, 1024, 4), (24576, 1024, 5), (2048, 1024, 32), (2048, 1024, 33),
+                                         (4096, 1024, 16), (4096, 1024, 17)])
+def test_either_side_of_a_line_bitwise(gpu, oracle, rows, cols, m):
+    import torch
+
+    from inferq_amd import synth as S
+
+    rng = np.random.default_rng([rows, cols, m])
+    w, mat = _mat(rows, cols, rng)
+    x = S.normal((m, cols), rng)
+    got = mat.forward(torch.from_numpy(x).to(gpu)).cpu().numpy()
+    assert_bitexact(got, oracle.matmul(S.Q8_0, w, rows, cols, x), f"[{rows} x {cols}] at {m} rows")
+
+
 @pytest.mark.parametrize("fill", [0x80, 0x7F, 0xFF, 0x00])
 def test_extreme_values_bitwise(gpu, oracle, fill):
     """Every weight byte -128, 127, -1 or 0 against rows that quantise to +-127."""
