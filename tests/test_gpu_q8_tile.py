@@ -110,31 +110,45 @@ def test_nonfinite_scales_as_the_lane_kernel(gpu, rows, cols, m):
     assert np.array_equal(bits(got)[ok], bits(ref)[ok])
 
 
-@pytest.mark.parametrize("tokens", [9, 33, 70])
+# past 48 tokens the shared expert runs on the many-row tiles, gate and up in one launch, SwiGLU inside down's
+# quantisation; hidden 1280: from 64 tokens only, its products apart below
+@pytest.mark.parametrize("tokens", [49, 64, 97])
 @pytest.mark.parametrize("hidden,inter", [(512, 256), (1280, 512)])
 def test_q8_shared_expert_wide_equals_narrow(gpu, tokens, hidden, inter):
-    """A Q8_0 shared expert run apart: gate and up in one launch and SwiGLU inside down's quantisation give each token
-    what a call of up to 8 tokens (the lane kernel and the SwiGLU launch) gives it, bit for bit."""
+    """Each token of a wide call gets, bit for bit, what calls of 8 tokens (the few-token kernels) give it and, with a
+    gate of exactly one half, what the lane kernel's products with SwiGLU in between add to the routed sum."""
     import torch
 
-    from inferq_amd import moe as M, synth as S
+    from inferq_amd import _lib, moe as M, qgemm as Q, synth as S
 
     rng = np.random.default_rng([tokens, hidden])
     gate = down = S.Q4_K
     layer = S.random_moe_layer(hidden, inter, 8, gate, down, rng)
-    for name, r, c in (("shared_gate", inter, hidden), ("shared_up", inter, hidden), ("shared_down", hidden, inter)):
+    shared = {"shared_gate": (inter, hidden), "shared_up": (inter, hidden), "shared_down": (hidden, inter)}
+    for name, (r, c) in shared.items():
         layer[name] = S.random_matrix(S.Q8_0, r, c, rng)
     t = {k: torch.from_numpy(v).to(gpu) for k, v in layer.items() if isinstance(v, np.ndarray)}
-    m = M.QuantizedMoeLayer(hidden, inter, 8, 2, gate, down, t["gate"], t["up"], t["down"], t["shared_gate"],
-                            t["shared_up"], t["shared_down"], t["selector"], shared_gate_dtype=S.Q8_0,
-                            shared_down_dtype=S.Q8_0)
     x = torch.from_numpy(S.normal((tokens, hidden), rng)).to(gpu)
     lg = torch.from_numpy(S.normal((tokens, 8), rng)).to(gpu)
-    wide, narrow = torch.empty_like(x), torch.empty_like(x)
-    m.forward_into(x, lg, wide)
-    for i in range(0, tokens, 8):
-        m.forward_into(x[i:i + 8].contiguous(), lg[i:i + 8].contiguous(), narrow[i:i + 8])
-    assert_bitexact(wide.cpu().numpy(), narrow.cpu().numpy(), f"{tokens} tokens")
+
+    def run(selector, step=tokens):
+        args = () if selector is None else (t["shared_gate"], t["shared_up"], t["shared_down"], selector)
+        m = M.QuantizedMoeLayer(hidden, inter, 8, 2, gate, down, t["gate"], t["up"], t["down"], *args,
+                                shared_gate_dtype=S.Q8_0, shared_down_dtype=S.Q8_0)
+        out = torch.empty_like(x)
+        for i in range(0, tokens, step):
+            m.forward_into(x[i:i + step].contiguous(), lg[i:i + step].contiguous(), out[i:i + step])
+        return out.cpu().numpy()
+
+    assert_bitexact(run(t["selector"]), run(t["selector"], 8), f"{tokens} tokens against 8")
+
+    mats = {k: Q.QuantizedMatrix.view(t[k], S.Q8_0, r, c) for k, (r, c) in shared.items()}
+    g, u = (mats[k].forward_via(x, _lib.PATH_LANES).cpu().numpy() for k in ("shared_gate", "shared_up"))
+    one = np.float32(1)
+    act = g / (one + np.exp(-g.astype(np.float64)).astype(np.float32)) * u
+    y = mats["shared_down"].forward_via(torch.from_numpy(act).to(gpu), _lib.PATH_LANES).cpu().numpy()
+    half = run(torch.zeros_like(t["selector"]))
+    assert_bitexact(half, run(None) + y * np.float32(0.5), f"{tokens} tokens against the lane kernel")
 
 
 # widths of one and several 256-value groups a wave, the widest (2048) and one past it, which runs as single products
