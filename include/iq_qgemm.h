@@ -172,7 +172,9 @@ int iq_matmul_reserve(iq_weight_t w, int64_t m, iq_stream_t stream);
 int iq_workspace_release(iq_stream_t stream);
 
 /* Device workspace bytes that serve every iq_matmul_ws call of up to m input
- * rows of W (any path): never less for more rows. */
+ * rows of W (any path): never less for more rows.  K-quant products of
+ * thousands of rows run pass by pass where the workspace given does not hold
+ * 548 bytes per 256 input values and 1 KiB. */
 size_t iq_matmul_workspace_size(iq_weight_t w, int64_t m);
 
 /* iq_matmul with a caller-provided device workspace (>= the size above). */

@@ -81,7 +81,8 @@ int current_device(int* dev) {
 
 }  // namespace
 
-int WsLease::acquire(size_t bytes, hipStream_t stream) {
+int WsLease::acquire(size_t bytes, hipStream_t stream, size_t least) {
+    least = std::min(bytes, least);
     int dev;
     if (int rc = current_device(&dev)) return rc;
     lock_ = std::unique_lock<std::mutex>(g_ws_mu);
@@ -96,12 +97,13 @@ int WsLease::acquire(size_t bytes, hipStream_t stream) {
         hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
         hipError_t e = hipStreamIsCapturing(stream, &cs);
         if (e != hipSuccess) return hip_fail(e, "hipStreamIsCapturing");
+        if (cs != hipStreamCaptureStatusNone && w->bytes >= least) return take(w->p, w->bytes);
         if (cs != hipStreamCaptureStatusNone)
             return fail(IQ_ERR_INVALID,
                         "the library workspace of this stream must grow to %zu bytes, which cannot happen during "
                         "graph capture: call iq_matmul_reserve (or make one eager call of the same size) on the "
                         "stream first, or pass a workspace (iq_matmul_ws)",
-                        bytes);
+                        least);
         // at least 1 MiB, and at least double the old size, so that a run of
         // growing calls retires few buffers
         size_t want = bytes < ((size_t)1 << 20) ? ((size_t)1 << 20) : bytes;
@@ -110,7 +112,16 @@ int WsLease::acquire(size_t bytes, hipStream_t stream) {
         e = hipMalloc(&np, want);
         if (e != hipSuccess) {
             (void)hipGetLastError();
-            if (want > bytes) e = hipMalloc(&np, want = bytes);  // doubling may not fit where the need does
+            // neither doubling nor a roomy workspace may fit where the need does
+            if (want > bytes) e = hipMalloc(&np, want = bytes);
+            if (e != hipSuccess && w->bytes >= least) {
+                (void)hipGetLastError();
+                return take(w->p, w->bytes);
+            }
+            if (e != hipSuccess && want > least) {
+                (void)hipGetLastError();
+                e = hipMalloc(&np, want = least);
+            }
             if (e != hipSuccess) {
                 (void)hipGetLastError();
                 return fail(IQ_ERR_OOM, "workspace allocation of %zu bytes failed: %s", want, hipGetErrorString(e));
@@ -122,8 +133,7 @@ int WsLease::acquire(size_t bytes, hipStream_t stream) {
         w->p = np;
         w->bytes = want;
     }
-    p_ = w->p;
-    return IQ_OK;
+    return take(w->p, w->bytes);
 }
 
 // Free the workspaces of `stream` on the current device (the live one and
@@ -253,8 +263,8 @@ int quantize_for(const iq_weight* w, const float* x, int64_t m, const ActView& a
     return IQ_OK;
 }
 
-// Device workspace a product of m rows needs (activation quantisation, and
-// for the int8-MFMA path its layouts and split-K partial tiles).
+// Device workspace a product of m rows cannot do without (activation
+// quantisation, and for the MFMA paths their layouts and split-K partial tiles).
 size_t matmul_ws_bytes(const iq_weight* w, int64_t m) {
     if (float_dtype(w->dtype)) return 0;  // the f32 product reads x as it is
     const size_t a = act_bytes(m, w->cols), p = prefill_workspace_size(view_of(w), m);
@@ -262,13 +272,18 @@ size_t matmul_ws_bytes(const iq_weight* w, int64_t m) {
     return std::max({a, p, d, q8_few_workspace(view_of(w), m)});
 }
 
-// The most any product of up to m rows needs: what a caller of narrower calls
-// too must hold.  The tile kernels' own needs fall where their plans change.
-size_t matmul_ws_upto(const iq_weight* w, int64_t m) {
-    if (float_dtype(w->dtype)) return 0;
+// The same for every product of up to m rows (the kernels' own needs fall
+// where their plans change), and what they use at most: a wide call takes
+// fewer passes with more than it needs.  Neither falls as m grows.
+static size_t matmul_ws_most(const iq_weight* w, int64_t m, size_t dense) {
     const WeightView v = view_of(w);
-    return std::max({act_bytes(m, w->cols), prefill_workspace_upto(v, m), dense_mfma_workspace_upto(v, m),
-                     q8_few_workspace(v, m)});
+    return std::max({act_bytes(m, w->cols), prefill_workspace_upto(v, m), dense, q8_few_workspace(v, m)});
+}
+size_t matmul_ws_upto(const iq_weight* w, int64_t m) {
+    return float_dtype(w->dtype) ? 0 : matmul_ws_most(w, m, dense_mfma_workspace_upto(view_of(w), m));
+}
+size_t matmul_ws_full(const iq_weight* w, int64_t m) {
+    return float_dtype(w->dtype) ? 0 : matmul_ws_most(w, m, dense_mfma_workspace_full(view_of(w), m));
 }
 
 // Greedy selection fused into the product (iq_matmul_argmax): 1 = one row
@@ -287,35 +302,29 @@ int64_t argmax_fused_parts(const iq_weight* w, int64_t m) {
     return f == 1 ? gemv_argmax_parts(view_of(w)) : f == 2 ? dense_argmax_parts(view_of(w)) : 0;
 }
 
-// Workspace of iq_matmul_argmax: the logits, then either the argmax
+// Workspace of an iq_matmul_argmax call: the logits, then either the argmax
 // partials and the product's own workspace or, fused, the pairs (keys,
-// then logits) and the product's workspace.
-size_t argmax_call_bytes(const iq_weight* w, int64_t m) {
+// then logits) and the product's workspace (product_bytes).
+size_t argmax_call_bytes(const iq_weight* w, int64_t m, size_t product_bytes) {
     const size_t yb = ((size_t)(m * w->rows) * 4 + 255) & ~(size_t)255;
     const size_t ab = (argmax_workspace_size(m, w->rows) + 255) & ~(size_t)255;
-    const size_t rest = ab + matmul_ws_bytes(w, m);
     const size_t P = (size_t)(m * argmax_fused_parts(w, m));
-    const size_t fused = P ? ((P * 8 + 255) & ~(size_t)255) + ((P * 4 + 255) & ~(size_t)255) + matmul_ws_bytes(w, m)
-                           : 0;
-    return yb + (rest > fused ? rest : fused);
+    return yb + std::max(ab, ((P * 8 + 255) & ~(size_t)255) + ((P * 4 + 255) & ~(size_t)255)) + product_bytes;
 }
 
-// The most any iq_matmul_argmax call of up to m rows needs (fused calls have
-// up to 8 rows).
-size_t argmax_call_upto(const iq_weight* w, int64_t m) {
-    const size_t yb = ((size_t)(m * w->rows) * 4 + 255) & ~(size_t)255;
-    size_t extra = (argmax_workspace_size(m, w->rows) + 255) & ~(size_t)255;
-    for (int64_t i = 1; i <= std::min<int64_t>(m, 8); i++) {
-        const size_t P = (size_t)(i * argmax_fused_parts(w, i));
-        extra = std::max(extra, ((P * 8 + 255) & ~(size_t)255) + ((P * 4 + 255) & ~(size_t)255));
-    }
-    return yb + extra + matmul_ws_upto(w, m);
+// What iq_matmul_argmax calls of up to m rows use at most (fused calls have up
+// to 8 rows).
+size_t argmax_call_full(const iq_weight* w, int64_t m) {
+    const size_t ws = matmul_ws_full(w, m);
+    size_t most = argmax_call_bytes(w, m, ws);
+    for (int64_t i = 1; i < std::min<int64_t>(m, 9); i++) most = std::max(most, argmax_call_bytes(w, i, ws));
+    return most;
 }
 
 // Kernel choice of a product (iq_matmul_via's path argument).  Every path
 // but IQ_PATH_PREFILL_TILES gives the reference's result bit for bit.
-hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, void* ws, int path, int32_t* isum,
-                       int32_t* msum, hipStream_t s) {
+hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, void* ws, size_t ws_bytes, int path,
+                       int32_t* isum, int32_t* msum, hipStream_t s) {
     const WeightView v = view_of(w);
     hipError_t e = hipErrorNotSupported;
     // F32 / BF16: one f32 product, no fixed kernel paths (the reference has
@@ -323,7 +332,7 @@ hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, 
     if (float_dtype(w->dtype))
         return path == IQ_PATH_AUTO && !isum ? launch_float_mm(v, x, w->cols, m, y, w->rows, s) : hipErrorNotSupported;
     if (path == IQ_PATH_AUTO) {
-        if (!isum && dense_mfma_supported(v, m)) e = launch_dense_mfma(v, x, w->cols, m, y, w->rows, ws, s);
+        if (!isum && dense_mfma_supported(v, m)) e = launch_dense_mfma(v, x, w->cols, m, y, w->rows, ws, ws_bytes, s);
         if (e == hipErrorNotSupported && !isum && q8_few_supported(v, m))
             e = launch_q8_few(v, x, w->cols, m, y, w->rows, ws, s);
         if (e == hipErrorNotSupported && !isum && q8_tile_supported(v, m))
@@ -332,7 +341,7 @@ hipError_t launch_path(const iq_weight* w, const float* x, int64_t m, float* y, 
     } else if (path == IQ_PATH_GEMV) {
         e = launch_gemv(v, x, w->cols, m, y, w->rows, s);
     } else if (path == IQ_PATH_LANE_MFMA) {
-        e = launch_dense_mfma_any(v, x, w->cols, m, y, w->rows, ws, s);
+        e = launch_dense_mfma_any(v, x, w->cols, m, y, w->rows, ws, ws_bytes, s);
     } else if (path == IQ_PATH_PREFILL_TILES) {
         e = launch_prefill(v, x, w->cols, m, y, w->rows, ws, nullptr, nullptr, s);
     }
@@ -366,12 +375,13 @@ int matmul_impl(const iq_weight* w, const float* x, int64_t m, float* y, void* w
     const size_t need = matmul_ws_bytes(w, m);
     WsLease lease;  // held until the launches below are enqueued
     if (!ws) {
-        if (int rc = lease.acquire(need, s)) return rc;
+        if (int rc = lease.acquire(std::max(need, matmul_ws_full(w, m)), s, need)) return rc;
         ws = lease.ptr();
+        ws_bytes = lease.bytes();
     } else if (ws_bytes < need) {
         return fail(IQ_ERR_SHAPE, "workspace of %zu bytes is smaller than the %zu bytes needed", ws_bytes, need);
     }
-    const hipError_t e = launch_path(w, x, m, y, ws, path, isum, msum, s);
+    const hipError_t e = launch_path(w, x, m, y, ws, ws_bytes, path, isum, msum, s);
     if (e == hipErrorNotSupported)
         return fail(IQ_ERR_DTYPE, "%s has no %s kernel for %lld input rows of a [%lld, %lld] matrix", dtype_name(w->dtype),
                     path_name(path), (long long)m, (long long)w->rows, (long long)w->cols);
@@ -522,7 +532,7 @@ IQ_API int iq_matmul_noalloc(iq_weight_t w, const float* x, int64_t m, float* y,
     if (int rc = scratch_ptr(&ws)) return rc;
     // every kernel of the dispatch writes the scratch it reads (quantised
     // activations, scales, sums) before reading it: nothing needs clearing
-    const hipError_t e = launch_path(w, x, m, y, ws, IQ_PATH_AUTO, nullptr, nullptr, (hipStream_t)stream);
+    const hipError_t e = launch_path(w, x, m, y, ws, kScratchBytes, IQ_PATH_AUTO, nullptr, nullptr, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "matmul launch");
     return IQ_OK;
 }
@@ -534,7 +544,7 @@ IQ_API int iq_matmul_reserve(iq_weight_t w, int64_t m, iq_stream_t stream) {
     if (m < 0) return fail(IQ_ERR_SHAPE, "negative input row count %lld", (long long)m);
     if (m == 0) return IQ_OK;
     // the widest of the entries that use the stream's workspace for W
-    const size_t need = std::max(matmul_ws_upto(w, m), m <= 65535 ? argmax_call_upto(w, m) : 0);
+    const size_t need = std::max(matmul_ws_full(w, m), m <= 65535 ? argmax_call_full(w, m) : 0);
     WsLease lease;
     return lease.acquire(need, (hipStream_t)stream);
 }
@@ -543,7 +553,9 @@ IQ_API int iq_workspace_release(iq_stream_t stream) { return release_workspace((
 
 IQ_API size_t iq_matmul_workspace_size(iq_weight_t w, int64_t m) {
     if (!w || m <= 0) return 0;
-    return matmul_ws_upto(w, m);
+    // up to what iq_matmul_noalloc has, the need itself, which tells whether it takes the call
+    const size_t need = matmul_ws_upto(w, m);
+    return need <= kScratchBytes ? need : matmul_ws_full(w, m);
 }
 
 IQ_API int iq_matmul_ws(iq_weight_t w, const float* x, int64_t m, float* y, void* workspace_ptr,
@@ -559,13 +571,12 @@ IQ_API int iq_matmul_host(iq_weight_t w, const float* x_host, int64_t m, float* 
     if (!x_host || !y_host) return fail(IQ_ERR_INVALID, "null input or output pointer");
     const size_t xb = (size_t)(m * w->cols) * 4, yb = (size_t)(m * w->rows) * 4;
     const size_t xo = 0, yo = (xb + 255) & ~(size_t)255, ao = yo + ((yb + 255) & ~(size_t)255);
-    const size_t need = ao + matmul_ws_bytes(w, m);
     WsLease lease;
-    if (int rc = lease.acquire(need, nullptr)) return rc;
+    if (int rc = lease.acquire(ao + matmul_ws_full(w, m), nullptr, ao + matmul_ws_bytes(w, m))) return rc;
     uint8_t* base = (uint8_t*)lease.ptr();
     hipError_t e = hipMemcpy(base + xo, x_host, xb, hipMemcpyHostToDevice);
     if (e != hipSuccess) return hip_fail(e, "hipMemcpy (input)");
-    if (int rc = matmul_impl(w, (const float*)(base + xo), m, (float*)(base + yo), base + ao, need - ao, IQ_PATH_AUTO,
+    if (int rc = matmul_impl(w, (const float*)(base + xo), m, (float*)(base + yo), base + ao, lease.bytes() - ao, IQ_PATH_AUTO,
                              nullptr, nullptr, nullptr))
         return rc;
     e = hipMemcpy(y_host, base + yo, yb, hipMemcpyDeviceToHost);
@@ -636,7 +647,9 @@ IQ_API int iq_matmul_argmax(iq_weight_t w, const float* x, int64_t m, int32_t* i
     const size_t yb = ((size_t)(m * w->rows) * 4 + 255) & ~(size_t)255;
     const size_t ab = (argmax_workspace_size(m, w->rows) + 255) & ~(size_t)255;
     WsLease lease;
-    if (int rc = lease.acquire(argmax_call_bytes(w, m), s)) return rc;
+    if (int rc = lease.acquire(argmax_call_bytes(w, m, matmul_ws_full(w, m)), s,
+                               argmax_call_bytes(w, m, matmul_ws_bytes(w, m))))
+        return rc;
     uint8_t* base = (uint8_t*)lease.ptr();
     float* y = (float*)base;
     if (const int f = argmax_fusion(w, m)) {
@@ -655,7 +668,7 @@ IQ_API int iq_matmul_argmax(iq_weight_t w, const float* x, int64_t m, int32_t* i
         if (e != hipSuccess) return hip_fail(e, "argmax launch");
         return IQ_OK;
     }
-    hipError_t e = launch_path(w, x, m, y, base + yb + ab, IQ_PATH_AUTO, nullptr, nullptr, s);
+    hipError_t e = launch_path(w, x, m, y, base + yb + ab, lease.bytes() - yb - ab, IQ_PATH_AUTO, nullptr, nullptr, s);
     if (e != hipSuccess) return hip_fail(e, "matmul launch");
     e = launch_argmax(y, m, w->rows, w->rows, idx, val, base + yb, s);
     if (e != hipSuccess) return hip_fail(e, "argmax launch");

@@ -39,19 +39,28 @@ class WsLease {
     WsLease() = default;
     WsLease(const WsLease&) = delete;
     WsLease& operator=(const WsLease&) = delete;
-    // Acquire at least `bytes` for `stream` on the current device.
-    int acquire(size_t bytes, hipStream_t stream);
+    // Acquire `bytes` for `stream` on the current device, or, where the
+    // workspace cannot grow to them (capture, memory), at least `least`.
+    int acquire(size_t bytes, hipStream_t stream, size_t least = SIZE_MAX);
     void* ptr() const { return p_; }
+    size_t bytes() const { return bytes_; }
 
   private:
+    int take(void* p, size_t bytes) {
+        p_ = p;
+        bytes_ = bytes;
+        return 0;
+    }
     std::unique_lock<std::mutex> lock_;
     void* p_ = nullptr;
+    size_t bytes_ = 0;
 };
 int check_weight(const iq_weight* w);
 // y = x . W^T through the dispatch (or a fixed path), with the caller's
 // workspace when ws is not null (ws_bytes >= matmul_ws_bytes(w, m)).
 size_t matmul_ws_bytes(const iq_weight* w, int64_t m);
 size_t matmul_ws_upto(const iq_weight* w, int64_t m);  // what any call of up to m rows needs
+size_t matmul_ws_full(const iq_weight* w, int64_t m);  // what any call of up to m rows uses at most
 int matmul_impl(const iq_weight* w, const float* x, int64_t m, float* y, void* ws, size_t ws_bytes, int path,
                 int32_t* isum, int32_t* msum, hipStream_t s);
 WeightView view_of(const iq_weight* w);

@@ -268,16 +268,25 @@ DmPlan dm_plan(const WeightView& w, int64_t m) {
     return P;
 }
 
-// Rows of the widest pass: as many as 16 MiB of workspace hold (3826 of
-// width 2048), what iq_matmul_noalloc has.  A wider call runs pass by pass
-// (rows are independent), its rows spread evenly.
-int64_t dm_max_pass_rows(const WeightView& w) {
-    const int64_t per_row = w.cols / 256 * (kMhBlock + 36);
-    return std::max<int64_t>((((int64_t)16 << 20) - 1024) / per_row, 1);
+// A call runs in one pass where its workspace allows: passes of 16 MiB (1913
+// rows of width 4096) leave a small matrix's launches short of workgroups
+// (Q6_K [512 x 8192] at 2048 rows, one pass / three of 16 MiB: 94 / 175 us).
+// 16 MiB, what iq_matmul_noalloc has, serve any call; a pass takes at most 256
+// MiB, which fill the GPU many times over (and which the tiles' 32-bit
+// activation offsets reach).
+constexpr size_t kDmPassLeast = (size_t)16 << 20, kDmPassMost = (size_t)256 << 20;
+
+size_t dm_row_bytes(const WeightView& w) { return (size_t)(w.cols / 256) * (kMhBlock + 36); }
+
+// Rows that `bytes` hold, plan alignment included (1024 bytes).
+int64_t dm_rows_in(const WeightView& w, size_t bytes) {
+    return std::max<int64_t>((int64_t)((bytes - 1024) / dm_row_bytes(w)), 1);
 }
 
-int64_t dm_pass_rows(const WeightView& w, int64_t m) {
-    const int64_t most = dm_max_pass_rows(w), passes = (m + most - 1) / most;
+// Rows of one pass with ws_bytes of workspace: the call's rows (they are
+// independent) spread evenly over as few passes as it takes.
+int64_t dm_pass_rows(const WeightView& w, int64_t m, size_t ws_bytes) {
+    const int64_t most = dm_rows_in(w, std::clamp(ws_bytes, kDmPassLeast, kDmPassMost)), passes = (m + most - 1) / most;
     return (m + passes - 1) / passes;
 }
 
@@ -361,21 +370,25 @@ bool dense_mfma_supported(const WeightView& w, int64_t m) {
 }
 
 size_t dense_mfma_workspace_any(const WeightView& w, int64_t m) {
-    return dm_layout_ok(w) && dm_rows_ok(w, m) ? dm_plan(w, dm_pass_rows(w, m)).total() : 0;
+    return dm_layout_ok(w) && dm_rows_ok(w, m) ? dm_plan(w, dm_pass_rows(w, m, kDmPassLeast)).total() : 0;
 }
 
-// A call just past the widest pass needs about half of that pass's bytes.
+// A call just past a pass of 16 MiB needs about half of that.
 size_t dense_mfma_workspace_upto(const WeightView& w, int64_t m) {
-    return m >= 1 && dm_layout_ok(w) ? dm_plan(w, std::min(m, dm_max_pass_rows(w))).total() : 0;
+    return m >= 1 && dm_layout_ok(w) ? dm_plan(w, std::min(m, dm_rows_in(w, kDmPassLeast))).total() : 0;
+}
+
+size_t dense_mfma_workspace_full(const WeightView& w, int64_t m) {
+    return m >= 1 && dm_layout_ok(w) ? (size_t)std::min(m, dm_rows_in(w, kDmPassMost)) * dm_row_bytes(w) + 1024 : 0;
 }
 
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                                 void* ws, hipStream_t s);
+                                 void* ws, size_t ws_bytes, hipStream_t s);
 
 hipError_t launch_dense_mfma(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                             void* ws, hipStream_t s) {
+                             void* ws, size_t ws_bytes, hipStream_t s) {
     if (!dense_mfma_supported(w, m)) return hipErrorNotSupported;
-    return launch_dense_mfma_any(w, x, ldx, m, y, ldy, ws, s);
+    return launch_dense_mfma_any(w, x, ldx, m, y, ldy, ws, ws_bytes, s);
 }
 
 // The split-K tile's choice: up to 8 rows on mid-size matrices of width
@@ -386,11 +399,11 @@ static bool dm_takes_sk(const WeightView& w, int64_t m) {
 }
 
 static hipError_t dense_run(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                            void* ws, uint64_t* amx_key, float* amx_val, hipStream_t s);
+                            void* ws, size_t ws_bytes, uint64_t* amx_key, float* amx_val, hipStream_t s);
 
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                                 void* ws, hipStream_t s) {
-    return dense_run(w, x, ldx, m, y, ldy, ws, nullptr, nullptr, s);
+                                 void* ws, size_t ws_bytes, hipStream_t s) {
+    return dense_run(w, x, ldx, m, y, ldy, ws, ws_bytes, nullptr, nullptr, s);
 }
 
 bool dense_argmax_supported(const WeightView& w, int64_t m) {
@@ -402,7 +415,7 @@ int64_t dense_argmax_parts(const WeightView& w) { return (w.rows + kMlCols - 1) 
 hipError_t launch_dense_argmax(const WeightView& w, const float* x, int64_t m, float* y, void* ws, uint64_t* keys,
                                float* vals, hipStream_t s) {
     if (!dense_argmax_supported(w, m) || !keys || !vals) return hipErrorNotSupported;
-    return dense_run(w, x, w.cols, m, y, w.rows, ws, keys, vals, s);
+    return dense_run(w, x, w.cols, m, y, w.rows, ws, kDmPassLeast, keys, vals, s);
 }
 
 template <int FMT>
@@ -456,10 +469,10 @@ static hipError_t dense_pass(const WeightView& w, const float* x, int64_t ldx, i
 }
 
 static hipError_t dense_run(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                            void* ws, uint64_t* amx_key, float* amx_val, hipStream_t s) {
+                            void* ws, size_t ws_bytes, uint64_t* amx_key, float* amx_val, hipStream_t s) {
     if (!dm_layout_ok(w) || !dm_rows_ok(w, m)) return hipErrorNotSupported;
     if (w.dtype == kQ5_K && m <= 8) return hipErrorNotSupported;  // a call, not a pass: the GEMV takes those
-    const int64_t pass = dm_pass_rows(w, m);
+    const int64_t pass = dm_pass_rows(w, m, ws_bytes);
     for (int64_t r = 0; r < m; r += pass)
         if (hipError_t e = dense_pass(w, x + r * ldx, ldx, std::min(pass, m - r), y + r * ldy, ldy, ws, amx_key, amx_val, s))
             return e;

@@ -79,15 +79,17 @@ hipError_t launch_prefill(const WeightView& w, const float* x, int64_t ldx, int6
 // says where the dispatch uses it (large matrices at 2..63 input rows, every
 // readable matrix from kPrefillMinRows rows); launch_dense_mfma_any runs it
 // at any row count on any matrix whose layout it can read.  Both quantise x
-// themselves into `ws` (at least dense_mfma_workspace_any bytes;
-// dense_mfma_workspace_upto: what any call of up to m rows needs).
+// themselves into `ws` (ws_bytes of it, at least dense_mfma_workspace_any;
+// dense_mfma_workspace_upto: what any call of up to m rows needs;
+// dense_mfma_workspace_full: what spares it a second pass).
 bool dense_mfma_supported(const WeightView& w, int64_t m);
 size_t dense_mfma_workspace_any(const WeightView& w, int64_t m);
 size_t dense_mfma_workspace_upto(const WeightView& w, int64_t m);
+size_t dense_mfma_workspace_full(const WeightView& w, int64_t m);
 hipError_t launch_dense_mfma(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                             void* ws, hipStream_t s);
+                             void* ws, size_t ws_bytes, hipStream_t s);
 hipError_t launch_dense_mfma_any(const WeightView& w, const float* x, int64_t ldx, int64_t m, float* y, int64_t ldy,
-                                 void* ws, hipStream_t s);
+                                 void* ws, size_t ws_bytes, hipStream_t s);
 
 // Q8_0 matrices at many input rows on f16 MFMA in the exact lane order
 // (iq_q8_tile.hip); quantises x itself into `ws` (at least act_bytes).

@@ -87,7 +87,7 @@ size_t carve(iq_moe* L, int m, uint8_t* base, MoeParams* p) {
         su = take((size_t)m * I * 4);
         sa = take((size_t)m * I * 4);
         so = take((size_t)m * H * 4);
-        smw_bytes = std::max({matmul_ws_upto(&L->sgate, m), matmul_ws_upto(&L->sup, m), matmul_ws_upto(&L->sdown, m)});
+        smw_bytes = std::max({matmul_ws_full(&L->sgate, m), matmul_ws_full(&L->sup, m), matmul_ws_full(&L->sdown, m)});
         smw = take(smw_bytes);
     }
     if (p) {

@@ -43,11 +43,11 @@ def test_extreme_integers_bitwise(gpu, oracle, dtype, fill):
 
 @pytest.mark.parametrize("dtype", [S.Q4_K, S.Q5_K, S.Q6_K])
 def test_passes_match_narrow_calls(gpu, dtype):
-    """A call past one pass (16 MiB of f16 activations) gives each row what a call of 64 rows gives it, also through
-    the allocation-free entry, whose 16 MiB it must not outgrow."""
+    """A call of more than 16 MiB of f16 activations gives each row what a call of 64 rows gives it, in one pass and
+    through the allocation-free entry, whose 16 MiB it must not outgrow."""
     from inferq_amd._lib import check, lib
 
-    rows, cols, m = 40, 8192, 1100  # at most 956 rows a pass: two of 550
+    rows, cols, m = 40, 8192, 1100  # 16 MiB hold 956 rows: two passes of 550
     rng = np.random.default_rng(dtype)
     mat = Q.QuantizedMatrix.upload(S.random_matrix(dtype, rows, cols, rng), dtype, rows, cols)
     x = torch.from_numpy(S.normal((m, cols), rng)).to(gpu)
