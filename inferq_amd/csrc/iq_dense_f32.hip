@@ -73,11 +73,13 @@ __global__ __launch_bounds__(64) void k_float_pair(const uint8_t* __restrict__ w
     };
     using std::integral_constant;
     while (k - h >= 64 * UM) pass(integral_constant<int, UM>{}, std::false_type{});
-    if (UM > 16 && k - h >= 64 * 16) pass(integral_constant<int, 16>{}, std::false_type{});
-    if (UM > 8 && k - h >= 64 * 8) pass(integral_constant<int, 8>{}, std::false_type{});
-    if (k - h > 64 * 4) pass(integral_constant<int, 8>{}, std::true_type{});
-    else if (k - h > 64) pass(integral_constant<int, 4>{}, std::true_type{});
-    else if (k - h > 0) pass(integral_constant<int, 1>{}, std::true_type{});
+    if (__builtin_expect(k > h, 0)) {  // out of the way of rows that have none: code to fetch is latency here
+        if (UM > 16 && k - h >= 64 * 16) pass(integral_constant<int, 16>{}, std::false_type{});
+        if (UM > 8 && k - h >= 64 * 8) pass(integral_constant<int, 8>{}, std::false_type{});
+        if (k - h > 64 * 4) pass(integral_constant<int, 8>{}, std::true_type{});
+        else if (k - h > 64) pass(integral_constant<int, 4>{}, std::true_type{});
+        else if (k - h > 0) pass(integral_constant<int, 1>{}, std::true_type{});
+    }
 #pragma unroll
     for (int i = 0; i < TT; i++) {
         float v = part[i];
