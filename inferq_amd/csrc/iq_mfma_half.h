@@ -12,9 +12,9 @@
 // lane, output and block before the chain's FMA (two in Q6_K's case), only
 // the FMA is left.  That matters because of what these cost on gfx950: with
 // two waves or more on a SIMD an f32 FMA issues in 2.5 cycles, a conversion,
-// shift-add or packed 16-bit operation in 4.2, a 16 x 16 MFMA in 18, and MFMA
-// and VALU issue hardly overlap.  Per 16 x 16 tile and Q4_K block that is
-// about 460 cycles against 900.
+// shift-add or packed 16-bit operation in 4.2, a 16 x 16 MFMA in 18, a third of
+// it under VALU issue.  Per 16 x 16 tile and Q4_K block that is about 460 cycles
+// of issue against 900 (what the kernel adds to them: see mh_product).
 #pragma once
 
 #include "iq_mfma_lanes.h"
@@ -63,10 +63,13 @@ __device__ __forceinline__ v2h_mh mh_both(float v) {
 // workgroup, the same result lanes), op.aq the f16 activations above (op.ldq
 // bytes a row).
 //
-// With two waves per SIMD (224 VGPRs at RT = 2) the loop is bound by what one
-// wave does in turn: [512 x 2048] -> 8192 Q4_K 77 -> 60 us, [512 x 4096] -> 2048
-// Q5_K 50 -> 38, [512 x 2048] -> 8192 Q6_K 84 -> 78 (its second MFMA and its
-// decode stay).
+// Bound by issue for about half of the time, for the rest by latency that two
+// waves per SIMD (224 VGPRs at RT = 2) do not cover: on [512 x 2048] -> 8192
+// Q4_K a tile and block take 1125 cycles of a SIMD, VALU active for 600 of them
+// (149 instructions), MFMA busy for 160, and a wave waits 28% of its time.
+// [512 x 2048] -> 8192 Q4_K 77 -> 60 us, [512 x 4096] -> 2048 Q5_K 50 -> 38, [512
+// x 2048] -> 8192 Q6_K 84 -> 78 (its second MFMA and its decode stay), against
+// the int8 form.
 // Splitting the eight lanes over two waves (128 VGPRs, four waves per SIMD)
 // measured 66-71 us for the Q4_K call, 64-row tiles 66: both decode or
 // address more per output than the occupancy returns.

@@ -100,7 +100,8 @@ struct QtStage {
 // rows 77 / 44 / 53; two tiles per wave with the MFMAs issued one step ahead,
 // two waves per SIMD, 61 / 54 / 56; a second stage of loads in flight the same;
 // every thread staging a quarter block (narrower loads, three times as many)
-// 68 / 45 / 52.
+// 68 / 45 / 52.  Four waves per SIMD leave 128 VGPRs, one too few: one is spilled
+// (8 bytes of scratch a lane).
 __global__ __launch_bounds__(512, 4) void k_qt_mm(QtArgs a) {
     constexpr int R = kQtRows, NT = 512;
     using L = QtStage;

@@ -61,8 +61,9 @@ def test_ties_non_finite_and_signed_zero(gpu):
 
 @pytest.mark.parametrize("n", [1, 255, 4096, 4097, 100003, 248320])
 def test_long_rows_match_the_rule(gpu, n):
-    """Chunk boundaries (4096 values per chunk), ragged tails, and maxima
-    placed at the first and last index and duplicated across chunks."""
+    """Chunk boundaries (1024 values per chunk up to 16 rows), ragged tails,
+    and maxima placed at the first and last index and duplicated across
+    chunks."""
     rng = np.random.default_rng(n)
     rows = rng.standard_normal((4, n), dtype=np.float32)
     rows[1, -1] = 100.0
@@ -72,6 +73,19 @@ def test_long_rows_match_the_rule(gpu, n):
         rows[3, 5000 % n] = np.nan
     idx, val = _gpu_argmax(gpu, rows)
     assert idx.tolist() == [ref_argmax(r) for r in rows]
+
+
+# up to 16 rows a chunk has 1024 values, from 17 on 4096
+@pytest.mark.parametrize("m", [16, 17])
+@pytest.mark.parametrize("n", [1024, 1025, 4096, 4097, 8200])
+def test_rows_on_either_side_of_the_chunk_sizes(gpu, m, n):
+    rng = np.random.default_rng([m, n])
+    rows = rng.standard_normal((m, n), dtype=np.float32)
+    rows[np.arange(m), rng.integers(0, n, m)] = 9.0
+    rows[0, -1], rows[1, 0], rows[2, [0, 1023, n - 1]], rows[3, [1022, 1023]] = 10.0, 10.0, 10.0, 10.0
+    idx, val = _gpu_argmax(gpu, rows)
+    assert idx.tolist() == [ref_argmax(r) for r in rows]
+    assert_bitexact(val, rows[np.arange(m), idx], "values")
 
 
 @pytest.fixture(scope="module")
