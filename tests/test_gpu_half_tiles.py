@@ -60,3 +60,27 @@ def test_passes_match_narrow_calls(gpu, dtype):
     check(lib().iq_matmul_noalloc(mat.handle, x.data_ptr(), m, y.data_ptr(), None))
     torch.cuda.synchronize()
     assert torch.equal(y.view(torch.int32), got.view(torch.int32))
+
+
+@pytest.mark.parametrize("rows,m", [(70, 64), (8256, 70)])
+@pytest.mark.parametrize("dtype", [S.Q4_K, S.Q5_K, S.Q6_K])
+def test_nonfinite_values_as_the_lane_kernel(gpu, dtype, rows, m):
+    """Infinities and NaN in rows and in block scales: NaN where the lane kernel has NaN, its bits elsewhere."""
+    from inferq_amd import _lib
+
+    cols = 512
+    rng = np.random.default_rng([dtype, m])
+    w = S.random_matrix(dtype, rows, cols, rng).reshape(rows, 2, -1)
+    d = 208 if dtype == S.Q6_K else 0
+    w[3, 1, d:d + 2] = np.array([0x7C00], np.uint16).view(np.uint8)  # inf
+    w[7, 0, d:d + 2] = np.array([0x7E00], np.uint16).view(np.uint8)  # NaN
+    if dtype != S.Q6_K:
+        w[9, 0, 2:4] = np.array([0xFC00], np.uint16).view(np.uint8)  # -inf, of the mins
+    x = S.normal((m, cols), rng)
+    x[2, 5], x[4, 300], x[6, 200] = np.inf, -np.inf, np.nan
+    mat = Q.QuantizedMatrix.upload(w.reshape(-1), dtype, rows, cols)
+    xd = torch.from_numpy(x).to(gpu)
+    got, ref = (mat.forward_via(xd, p).cpu().numpy() for p in (_lib.PATH_AUTO, _lib.PATH_LANES))
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    ok = ~np.isnan(ref)
+    assert np.array_equal(got[ok].view(np.uint32), ref[ok].view(np.uint32))
