@@ -26,6 +26,7 @@ struct iq_moe {
     std::mutex mu;
     void* ws = nullptr;
     size_t ws_bytes = 0;
+    size_t shared_ws_bytes = 0;  // of them for a shared expert's products (shared_need at ws_m)
     int ws_m = 0;
     // Workspaces replaced by a larger one.  A graph captured earlier still
     // holds their addresses, so they stay allocated until the handle is
@@ -41,8 +42,15 @@ constexpr size_t a256(size_t n) { return (n + 255) & ~(size_t)255; }
 
 int64_t row_bytes_of(int dtype, int64_t cols) { return cols / block_elems(dtype) * block_bytes(dtype); }
 
-// Carve the per-call workspace for m tokens; returns its size when base is null.
-size_t carve(iq_moe* L, int m, uint8_t* base, MoeParams* p) {
+// Workspace of a shared expert's products run apart, for calls of up to m tokens.
+size_t shared_need(const iq_moe* L, int m) {
+    if (!L->shared_apart) return 0;
+    return std::max({matmul_ws_full(&L->sgate, m), matmul_ws_full(&L->sup, m), matmul_ws_full(&L->sdown, m)});
+}
+
+// Carve the per-call workspace for m tokens, smw_bytes of it shared_need(L,
+// m); returns its size when base is null.
+size_t carve(iq_moe* L, int m, size_t smw_bytes, uint8_t* base, MoeParams* p) {
     const int64_t K = L->layer.K, H = L->layer.H, I = L->layer.I;
     const int64_t na = m * K, gmax = na + 1, P = na + m;
     const int64_t ngI = (I + 255) / 256;
@@ -81,13 +89,11 @@ size_t carve(iq_moe* L, int m, uint8_t* base, MoeParams* p) {
     // the shared expert run apart: gate, up and SwiGLU rows [m x I], its
     // output [m x H] and the products' workspace
     uint8_t *sg = nullptr, *su = nullptr, *sa = nullptr, *so = nullptr, *smw = nullptr;
-    size_t smw_bytes = 0;
     if (L->shared_apart) {
         sg = take((size_t)m * I * 4);
         su = take((size_t)m * I * 4);
         sa = take((size_t)m * I * 4);
         so = take((size_t)m * H * 4);
-        smw_bytes = std::max({matmul_ws_full(&L->sgate, m), matmul_ws_full(&L->sup, m), matmul_ws_full(&L->sdown, m)});
         smw = take(smw_bytes);
     }
     if (p) {
@@ -153,7 +159,7 @@ int grow_workspace(iq_moe* L, int m, hipStream_t s, bool at_create = false) {
                     "the MoE workspace must grow to %d tokens, which cannot happen during graph capture: call "
                     "iq_moe_reserve (or make one eager call of at least this many tokens) on the handle first",
                     m);
-    const size_t bytes = carve(L, m, nullptr, nullptr);
+    const size_t shared = shared_need(L, m), bytes = carve(L, m, shared, nullptr, nullptr);
     void* ws = nullptr;
     e = hipMalloc(&ws, bytes);
     if (e != hipSuccess) {
@@ -168,6 +174,7 @@ int grow_workspace(iq_moe* L, int m, hipStream_t s, bool at_create = false) {
     if (L->ws) L->retired.push_back(L->ws);
     L->ws = ws;
     L->ws_bytes = bytes;
+    L->shared_ws_bytes = shared;
     L->ws_m = m;
     return IQ_OK;
 }
@@ -299,7 +306,7 @@ static int moe_slice(iq_moe_t L, const float* x, const float* logits, const floa
                      int32_t* experts_out, float* weights_out, void* const* events, hipStream_t s) {
     if (int rc = grow_workspace(L, (int)m, s)) return rc;
     MoeParams p = L->layer;
-    carve(L, L->ws_m, (uint8_t*)L->ws, &p);
+    carve(L, L->ws_m, L->shared_ws_bytes, (uint8_t*)L->ws, &p);
     // carve() sized the views for ws_m tokens; the call uses m
     p.xq.m = (int)m;
     p.x = x;
